@@ -87,7 +87,8 @@ KERNEL_NAMES = [
     (r"lse_merge_kernel", "lse_merge"),
     (r"merge_kernel", "merge_rows"),
     (r"finalize_kernel", "finalize_metrics"),
-    (r"row_parts_kernel", "row_parts"),
+    (r"row_parts_kernel|emit_rows_kernel", "row_parts"),
+    (r"emit_tiles_kernel", "head_emit"),
     (r"accept_rows_kernel", "accept_rows"),
     (r"sum_partials_kernel", "dprev_reduce"),
     (r"gather_rows_kernel", "markov_gather"),
@@ -597,7 +598,7 @@ def workload_head(device, args, which):
         return metrics, dh
 
     gemm = 2.0 * n * v * d
-    kernel_flops = {"head_stats": gemm, "head_emit": gemm, "dh_gemm": gemm}
+    kernel_flops = {"head_stats": gemm, "dh_gemm": gemm}
     rows2 = n
     if skip:
         # pass 2 and the dh GEMM run on the rows whose dl is not all zero: here the supervised
@@ -605,9 +606,11 @@ def workload_head(device, args, which):
         rows2 = int(((slots.valid.reshape(-1) != 0) | (slots.weights.reshape(-1) != 0)).sum())
         kernel_flops = {"head_stats": gemm, "head_emit": 2.0 * rows2 * v * d, "dh_gemm": 2.0 * rows2 * v * d}
     kernel_fp8_flops = {"fp8_head_gemm": gemm} if fp8 is not None else {}
-    # byte streams of the epilogues (for the per-kernel GB/s report): pass 1 reads
-    # Markov + teacher, pass 2 also writes dl; the dh GEMM reads dl
-    kernel_bytes = {"head_stats": 4 * n * v, "head_emit": 6 * n * v, "dh_gemm": 2 * n * v}
+    # byte streams (for the per-kernel GB/s report): pass 1 reads Markov + teacher and writes
+    # its fp32 values, pass 2 reads them and the teacher and writes dl; the dh GEMM reads dl
+    kernel_bytes = {"head_stats": 8 * n * v, "head_emit": 8 * n * v, "dh_gemm": 2 * n * v}
+    if skip:   # pass 1 keeps nothing, pass 2 runs the GEMM on its rows
+        kernel_bytes = {"head_stats": 4 * n * v, "head_emit": 6 * rows2 * v, "dh_gemm": 2 * rows2 * v}
 
     def cpu_baseline(rows):
         import numpy as np
@@ -679,7 +682,7 @@ def workload_head(device, args, which):
 
     executed = gemm + 4.0 * rows2 * v * d if skip else None   # pass 1 on N rows, pass 2 and dh on rows2
     return dict(step=step, n=n, per_slot_bytes=None, per_slot_flops=4.0 * v * d, kernel_bytes=kernel_bytes,
-                executed_flops_per_step=executed,
+                stream_kernels=("head_emit",), executed_flops_per_step=executed,
                 kernel_flops=kernel_flops, kernel_fp8_flops=kernel_fp8_flops, cpu_baseline=cpu_baseline,
                 config=config, dtype="bf16" if fp8 is None else "bf16+fp8", ceilings=ceilings,
                 per_slot_fp8_flops=2.0 * v * d if fp8 is not None else None,
@@ -737,8 +740,8 @@ def workload_c2x(device, args):
         return metrics, dx
 
     gemm_k = 2.0 * n * v * (d + r)
-    kernel_flops = {"head_stats": gemm_k, "head_emit": gemm_k, "dh_gemm": gemm_k, "markov_dw2": 2.0 * n * v * r}
-    kernel_bytes = {"head_stats": 2 * n * v, "head_emit": 4 * n * v, "dh_gemm": 2 * n * v,
+    kernel_flops = {"head_stats": gemm_k, "dh_gemm": gemm_k, "markov_dw2": 2.0 * n * v * r}
+    kernel_bytes = {"head_stats": 6 * n * v, "head_emit": 8 * n * v, "dh_gemm": 2 * n * v,
                     "markov_dw2": 2 * n * v, "rms_norm_fwd": 6 * n * d}
 
     def cpu_baseline(rows):
@@ -782,6 +785,7 @@ def workload_c2x(device, args):
               "global_batch": n, "seq_len": None, "parallelism": "single GPU"}
     return dict(step=step, n=n, per_slot_bytes=None, per_slot_flops=4.0 * v * d + 6.0 * v * r,
                 kernel_bytes=kernel_bytes, kernel_flops=kernel_flops, kernel_fp8_flops={},
+                stream_kernels=("head_emit",),
                 cpu_baseline=cpu_baseline, config=config, dtype="bf16", per_slot_fp8_flops=None,
                 inputs={"pre_norm_hidden": x, "lm_head_weight": weight, "teacher_logits": teacher,
                         "previous": prev, "markov_w1": w1, "markov_w2": w2, "weights": slots.weights,
@@ -921,7 +925,9 @@ def measure(wl, args, config_name):
     ms_per_step = gpu_ms / args.steps
     n = wl["n"]
     value = n * args.steps / (gpu_ms / 1e3)
-    kernels = {name: {"launches": c, "mean_ms": tot / max(c, 1), "window": "timed"}
+    # a workload's per-kernel work is a step's: a kernel launched for each window of rows has
+    # it spread over several launches
+    kernels = {name: {"launches": c, "mean_ms": tot / max(c, 1), "step_ms": tot / args.steps, "window": "timed"}
                for name, (c, tot) in kt.times.items()}
     # the short kernels' means from a few more steps after the timed window, every launch timed
     detail_steps = max(3, args.steps // 4)
@@ -931,10 +937,11 @@ def measure(wl, args, config_name):
         torch.cuda.synchronize()
     for name, (c, tot) in kd.times.items():
         if name not in kernels:
-            kernels[name] = {"launches": c, "mean_ms": tot / max(c, 1), "window": f"{detail_steps} steps after"}
+            kernels[name] = {"launches": c, "mean_ms": tot / max(c, 1), "step_ms": tot / detail_steps,
+                             "window": f"{detail_steps} steps after"}
 
     def roofline(kernel):
-        k_ms = kernels[kernel]["mean_ms"]
+        k_ms, launch_ms = kernels[kernel]["step_ms"], kernels[kernel]["mean_ms"]
         if kernel in wl["kernel_flops"] or kernel in fp8_flops:
             fp8 = kernel in fp8_flops
             peak = FP8_PEAK_TFLOPS if fp8 else BF16_PEAK_TFLOPS
@@ -946,14 +953,14 @@ def measure(wl, args, config_name):
             roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": achieved / HBM_PEAK_GBS}
         roof["kernel"] = kernel
-        roof["kernel_mean_ms"] = k_ms
+        roof["kernel_mean_ms"] = launch_ms
         tr = committed_traffic(config_name, kernel)
         roof["traffic"] = tr[0] if tr else None
         if tr:
             roof["traffic_source"] = tr[1]
             # the bytes the kernel moves (counters), over this run's mean launch time: the
             # executed HBM rate beside the algorithmic one above
-            roof["traffic_GBs"] = tr[0] / (k_ms / 1e3) / 1e9
+            roof["traffic_GBs"] = tr[0] / (launch_ms / 1e3) / 1e9
             roof["traffic_frac_hbm"] = roof["traffic_GBs"] / HBM_PEAK_GBS
         mf = committed_mfma(config_name, kernel)
         if mf:
@@ -964,12 +971,12 @@ def measure(wl, args, config_name):
     roof = roofline(dominant)
     for name, info in kernels.items():
         if name in wl["kernel_bytes"]:
-            info["algorithmic_GBs"] = wl["kernel_bytes"][name] / (info["mean_ms"] / 1e3) / 1e9
+            info["algorithmic_GBs"] = wl["kernel_bytes"][name] / (info["step_ms"] / 1e3) / 1e9
         if name in wl["kernel_flops"]:
-            info["algorithmic_TFLOPs"] = wl["kernel_flops"][name] / (info["mean_ms"] / 1e3) / 1e12
+            info["algorithmic_TFLOPs"] = wl["kernel_flops"][name] / (info["step_ms"] / 1e3) / 1e12
             info["mfma_frac"] = info["algorithmic_TFLOPs"] / BF16_PEAK_TFLOPS
         if name in fp8_flops:
-            info["algorithmic_TFLOPs"] = fp8_flops[name] / (info["mean_ms"] / 1e3) / 1e12
+            info["algorithmic_TFLOPs"] = fp8_flops[name] / (info["step_ms"] / 1e3) / 1e12
             info["mfma_frac_fp8"] = info["algorithmic_TFLOPs"] / FP8_PEAK_TFLOPS
     step_roof = {}
     if wl["per_slot_bytes"]:

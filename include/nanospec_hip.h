@@ -63,12 +63,13 @@ extern "C" {
 #define NS_ENULL (-5)      /* required pointer is NULL */
 
 #define NS_WS_LOGITS 0   /* ns_ce_kl_logits_fwd */
-#define NS_WS_LMHEAD 1   /* ns_lmhead_ce_kl_fwd */
+#define NS_WS_LMHEAD 1   /* ns_lmhead_ce_kl_fwd: pass 2 reads pass 1's values (at most 2 GiB and partials) */
 #define NS_WS_LMHEAD_BWD 2 /* ns_lmhead_bwd */
 #define NS_WS_FP8 3      /* ns_fp8_teacher_logits */
 #define NS_WS_RMS_NORM_BWD 4     /* ns_rms_norm_bwd (v ignored) */
 #define NS_WS_LMHEAD_NORM_BWD 5  /* ns_lmhead_norm_bwd */
 #define NS_WS_TEACHER_LOGITS 6   /* ns_lmhead_teacher_logits with lse (d ignored) */
+#define NS_WS_LMHEAD_MIN 7       /* what every fused-head entry accepts (d ignored): pass 2 runs the GEMM again */
 
 typedef struct ihipStream_t* ns_stream_t; /* == hipStream_t */
 
@@ -126,10 +127,12 @@ int ns_ce_kl_logits_bwd(const void* z, int z_dtype, int64_t ldz, const void* u, 
                         ns_stream_t stream);
 
 /* Fused LM head + objective forward (train.py:272-279 -> objective.py:49-67):
- * z = hidden . weight^T (+ markov) is formed tile by tile on bf16 MFMA and never
- * stored; pass 1 folds (max, sum-exp) of z and the teacher row and A = sum t(u - z);
- * pass 2 recomputes z and emits the accept rate and, when dl is not NULL,
- * dl = (w * inv_acc)[(c_ce + c_kl) p - c_kl t - c_ce e_y] as bf16.
+ * z = hidden . weight^T (+ markov) is formed tile by tile on bf16 MFMA, in windows of rows
+ * (at most 2 GiB of z is held at a time); pass 1 folds (max, sum-exp) of z and the teacher row and
+ * A = sum t(u - z); pass 2 emits the accept rate and, when dl is not NULL,
+ * dl = (w * inv_acc)[(c_ce + c_kl) p - c_kl t - c_ce e_y] as bf16, from the window's fp32 z
+ * kept in the workspace (NS_WS_LMHEAD: at most 2 GiB and the partials) or, with a smaller
+ * workspace (NS_WS_LMHEAD_MIN), from z formed again: the same bits.
  * hidden [N, d] bf16, weight [V, d] bf16 (the frozen LM head), markov [N, V] bf16
  * or NULL, teacher [N, V] (t_dtype), dl [N, V] bf16 or NULL.
  * Requires d % 64 == 0, V % 8 == 0, 16-byte aligned rows, n % k == 0. */

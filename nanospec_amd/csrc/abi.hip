@@ -95,6 +95,8 @@ size_t ns_workspace_bytes(int kind, int64_t n, int64_t v, int64_t d) {
       return ns::lmhead_bwd_workspace_bytes(n, v, d, 0, true);
     case NS_WS_TEACHER_LOGITS:
       return ns::lmhead_linear_lse_workspace_bytes(n, v);
+    case NS_WS_LMHEAD_MIN:
+      return ns::lmhead_min_workspace_bytes(n, v);
     default:
       return 0;
   }
@@ -198,7 +200,8 @@ int check_head_inputs(const void* hidden, int64_t ldh, const void* weight, int64
     if (v * factors->ldw1 * 2 >= (int64_t(1) << 32))
       return fail(NS_EINVAL, "w1 spans %lld bytes; at most 4 GiB", (long long)(v * factors->ldw1 * 2));
   }
-  const size_t need = ns::lmhead_workspace_bytes(n, v, d);
+  // (a smaller one than ns_workspace_bytes' takes pass 2 through the GEMM again)
+  const size_t need = ns::lmhead_required_bytes(n, v);
   if (n > 0 && (!workspace || workspace_bytes < need))
     return fail(NS_EWORKSPACE, "workspace of %zu bytes required (got %zu)", need, workspace_bytes);
   if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return fail(NS_EALIGN, "workspace must be 256-byte aligned");
@@ -220,7 +223,7 @@ int lmhead_fwd_checked(const void* hidden, int64_t ldh, const void* weight, int6
   ns::SlotArgs a{labels, weights, valid, n, k, c_ce, c_kl, inv_acc};
   const ns::TeacherSpec ts{targs ? targs->rows : nullptr, nt, targs ? targs->lse : nullptr};
   return hip_status(ns::lmhead_forward(hidden, ldh, weight, ldw, markov, ldm, factors, teacher, t_dtype, ldt, d, v,
-                                       a, &ts, dl, ldd, row_stats, metrics, workspace,
+                                       a, &ts, dl, ldd, row_stats, metrics, workspace, workspace_bytes,
                                        reinterpret_cast<hipStream_t>(stream)),
                     name);
 }
@@ -256,7 +259,7 @@ int ns_lmhead_ce_kl_fwd_part(int part, const void* hidden, int64_t ldh, const vo
   ns::SlotArgs a{labels, weights, nullptr, n, 1, c_ce, c_kl, inv_acc};
   const ns::TeacherSpec ts{teacher_args ? teacher_args->rows : nullptr, nt, teacher_args ? teacher_args->lse : nullptr};
   return hip_status(ns::lmhead_forward(hidden, ldh, weight, ldw, markov, ldm, nullptr, teacher, t_dtype, ldt, d, v, a,
-                                       &ts, dl, ldd, row_stats, nullptr, workspace,
+                                       &ts, dl, ldd, row_stats, nullptr, workspace, workspace_bytes,
                                        reinterpret_cast<hipStream_t>(stream),
                                        part == NS_PART_STATS ? ns::kHeadStats : ns::kHeadEmit),
                     "ns_lmhead_ce_kl_fwd_part");
@@ -335,7 +338,7 @@ int ns_lmhead_ce_kl_fwd_noalloc(const void* hidden, int64_t ldh, const void* wei
                                 const uint8_t* valid, int64_t n, int64_t d, int64_t v, int64_t k, float c_ce,
                                 float c_kl, float inv_acc, void* dl, int64_t ldd, float* row_stats, float* metrics,
                                 ns_stream_t stream) {
-  const size_t need = n > 0 && v > 0 ? ns::lmhead_workspace_bytes(n, v, d) : 0;
+  const size_t need = n > 0 && v > 0 ? ns::lmhead_required_bytes(n, v) : 0;
   if (need > kNoAllocScratchBytes)
     return fail(NS_EWORKSPACE,
                 "ns_lmhead_ce_kl_fwd_noalloc: n = %lld, v = %lld need %zu bytes of scratch; its static scratch "
@@ -382,7 +385,7 @@ int ns_lmhead_ce_kl_bwd(const void* hidden, int64_t ldh, const void* weight, int
   ns::SlotArgs a{labels, weights, nullptr, n, 1, c_ce, c_kl, inv_acc};
   const ns::TeacherSpec ts{teacher_args ? teacher_args->rows : nullptr, nt, teacher_args ? teacher_args->lse : nullptr};
   return hip_status(ns::lmhead_emit_dlogits(hidden, ldh, weight, ldw, markov, ldm, factors, teacher, t_dtype, ldt, d,
-                                            v, a, &ts, row_stats, dl, ldd, workspace,
+                                            v, a, &ts, row_stats, dl, ldd, workspace, workspace_bytes,
                                             reinterpret_cast<hipStream_t>(stream)),
                     "ns_lmhead_ce_kl_bwd");
 }

@@ -1,15 +1,19 @@
 // Fused LM head + draft objective on bf16 MFMA (gfx950, v_mfma_f32_32x32x16_bf16).
 //
-// Forward (nanospec/train.py:272-279 + objective.py:49-67), never storing logits:
+// Forward (nanospec/train.py:272-279 + objective.py:49-67), over windows of rows, so that at
+// most 2 GiB of logits are held at a time, whatever N is:
 //   z^T tile = W_lm[v-tile] . hidden[t-tile]^T   (vocab on the MFMA M axis, tokens on N)
 //   pass 1 ("stats"): epilogue adds the Markov tile, reads the teacher tile and folds
 //     (max, sum-exp) of z and u plus A = sum exp(u - m_u)(u - z) into per-token running
 //     state kept in LDS across the workgroup's vocab range -> RowPart partials; the lane
 //     that owns (token, label) writes z_label.
 //   merge (shared with the logits path): LSE_z, LSE_u, CE, KL per token.
-//   pass 2 ("emit"): recomputes the z tile, p = exp(z - LSE_z), t = exp(u - LSE_u),
-//     accumulates sum min(p, t) and writes dl = (w/acc)[(c_ce + c_kl) p - c_kl t - c_ce e_y]
-//     as bf16.
+//   pass 2 ("emit"): p = exp(z - LSE_z), t = exp(u - LSE_u), accumulates sum min(p, t) and
+//     writes dl = (w/acc)[(c_ce + c_kl) p - c_kl t - c_ce e_y] as bf16.  With workspace for
+//     one window's values pass 1 keeps its fp32 tiles there (kKeepZ: 4 bytes per entry written
+//     beside the epilogue, 3% of pass 1) and pass 2 streams over them (emit.hip); without, it
+//     runs the GEMM again (head_kernel<EMIT>).  At N = 4096, d = 5120, V = 248,320: both passes
+//     16.5 ms with the GEMM twice, 10.4 ms with the values kept (two windows).
 // Backward (train.py:302): dh = dl . W_lm as a long-K (K = V) split-K MFMA GEMM with a
 // fixed-order fp32 reduction of the split partials.
 //
@@ -455,12 +459,14 @@ struct HeadParams {
   int64_t nh;
   // launches by round (launch_head): this launch's first workgroup id and the whole grid; 0: one launch
   int wg0, wg_total;
+  float* z;                 // kKeepZ: pass 1's tile values, [tt][vt] tiles of kZTile (ns_internal.h)
 };
 
 enum { MODE_STATS = 0, MODE_EMIT = 1, MODE_STORE = 2 };
 // head_kernel variants: the teacher's log-normaliser is given (STATS / EMIT), the stored
-// values' log-sum-exp partials are formed (STORE)
-enum { kTeacherLse = 1, kStoreLse = 2 };
+// values' log-sum-exp partials are formed (STORE), the tile's values are kept for the
+// streaming second pass (STATS)
+enum { kTeacherLse = 1, kStoreLse = 2, kKeepZ = 4 };
 
 // Head-kernel LDS beyond the GEMM stages: per-token running state and per-token
 // constants of the workgroup's 256 tokens (they persist across vocab tiles).  The state
@@ -476,21 +482,6 @@ constexpr int kTbadOff = kTrowOff + 256 * 4;        // [256] uint8: teacher (STO
 constexpr int kHrowOff = kTbadOff + 256;            // [256] int32 gathered B rows (MODE_STORE)
 constexpr int kHeadLdsBytes = kHrowOff + 256 * 4;
 static_assert(kHeadLdsBytes <= 160 * 1024, "head kernel LDS");
-
-// Lanes l and l ^ 32 hold the same token (vocab entries 4 h .. 4 h + 3 of each 8-entry
-// chunk, h = l / 32).  v_permlane32_swap hands every lane both lanes' values in the same
-// order, so a symmetric merge of the two leaves identical bits in both.
-__device__ __forceinline__ void half_pair(float x, float& a, float& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  a = __uint_as_float(r[0]);
-  b = __uint_as_float(r[1]);
-}
-
-__device__ __forceinline__ float half_sum(float x) {
-  float a, b;
-  half_pair(x, a, b);
-  return a + b;
-}
 
 __device__ __forceinline__ PairState half_merge(const PairState& s) {
   PairState a, b;
@@ -744,6 +735,8 @@ struct StreamTail {
 
 typedef uint32_t u32x2v_t __attribute__((ext_vector_type(2)));
 
+constexpr int kZAux = 2;   // kept tile values: written once, read once by a later kernel (nt)
+
 // Objective epilogue of one 256 x 256 tile (layout above).  Each lane folds its token's
 // 64 entries per step locally, the two lanes of a token combine (half_merge / half_sum),
 // and the lane of the lower half folds the result into the token's running state for
@@ -909,6 +902,20 @@ __device__ __forceinline__ void epilogue_tile(const HeadParams& p, lds_t* lds, c
         }
       }
       const bool any = FULL || okc[0];
+      if (MODE == MODE_STATS && (FLAGS & kKeepZ)) {
+        // The half-step's values as they lie in the registers: 1 KB per chunk, lane after
+        // lane (emit.hip reads them with the same lanes).  A block of 32 tokens past N is
+        // dropped by the buffer's range (length 0).
+        const __amdgpu_buffer_rsrc_t zrs = __builtin_amdgcn_make_buffer_rsrc(
+            p.z + ((t0 / BN) * p.vt + v0 / BM) * kZTile, 0, t0 + wn * 128 + 32 * s < p.n ? (int)(kZTile * 4) : 0,
+            0x00020000);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const f32x4_t zc = {z[4 * c], z[4 * c + 1], z[4 * c + 2], z[4 * c + 3]};
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, zc), zrs, ln * 16,
+                                                 ((s * 4 + wv) * 16 + 8 * hs + c) * 1024, kZAux);
+        }
+      }
       if (MODE == MODE_STATS) {
         auto next2 = [&](int g) {
           next(2 * (4 * hs + g));
@@ -1327,6 +1334,35 @@ HeadPlan head_plan(int64_t n, int64_t v) {
   return pl;
 }
 
+// The forward runs over windows of whole token tiles, so that the tile values pass 1 keeps for
+// pass 2 fit kZWindowBytes whatever N is (2,048 rows at V = 248,320): the
+// [N, V] logits beyond that never exist together.  Windows are of even size (all but the last the
+// same); pass 2 without kept values follows the same windows, so that both ways add every sum
+// in the same order.  At N = 4096 two windows cost pass 1 2% (31 vocab tiles a workgroup twice,
+// for 61 once).
+constexpr int64_t kZWindowBytes = int64_t(2) << 30;
+
+int64_t window_rows(int64_t n, int64_t v) {
+  const int64_t vt = (v + BM - 1) / BM, tt = (n + BN - 1) / BN;
+  if (tt == 0 || vt == 0) return n;
+  int64_t most = kZWindowBytes / (vt * kZTile * 4);   // token tiles
+  if (most >= 4) most -= most % 4;                    // whole XCD blocks (4 x 8)
+  if (most < 1) most = 1;
+  const int64_t windows = (tt + most - 1) / most;
+  return (tt + windows - 1) / windows * BN;
+}
+
+// Whether pass 2 reads pass 1's tile values (4 bytes written and 4 read per entry) rather than
+// running the GEMM again (2 d operations per entry).  Both passes in microseconds, kept against
+// GEMM again, V = 248,320 unless said: N = 3500: d = 128 2557 / 2219, 256 2761 / 2663, 384
+// 2972 / 3030, 512 3296 / 3452; N = 448: 128 360 / 359, 256 382 / 417; N = 2048, V = 32,000:
+// 128 198 / 183, 256 210 / 211; N = 56: 128 147 / 200; N = 64, V = 8192, d = 64: 40 / 55.  The
+// fewer the values, the more of them the Infinity Cache (256 MB) still holds for pass 2.
+bool keeps_tiles(int64_t n, int64_t v, int64_t d) {
+  const int64_t entries = n * v;
+  return d >= (entries <= (int64_t(1) << 25) ? 64 : entries <= (int64_t(1) << 27) ? 192 : 320);
+}
+
 struct HeadWs {
   RowPart* part1;
   float* parta;
@@ -1334,10 +1370,10 @@ struct HeadWs {
   float* partk;   // pass-2 KL partials (teacher log-normaliser given)
 };
 
-size_t head_ws_layout(int64_t n, int64_t v, void* base, HeadWs* out) {
-  const HeadPlan pl = head_plan(n, v);
-  const size_t b1 = align_up((size_t)n * pl.splits * sizeof(RowPart), 256);
-  const size_t b2 = align_up((size_t)n * pl.splits * sizeof(float), 256);
+// One window's partials.
+size_t window_ws_layout(int64_t n, int splits, void* base, HeadWs* out) {
+  const size_t b1 = align_up((size_t)n * splits * sizeof(RowPart), 256);
+  const size_t b2 = align_up((size_t)n * splits * sizeof(float), 256);
   const size_t b3 = align_up((size_t)n * sizeof(float), 256);
   if (out) {
     char* c = static_cast<char*>(base);
@@ -1347,6 +1383,27 @@ size_t head_ws_layout(int64_t n, int64_t v, void* base, HeadWs* out) {
     out->partk = reinterpret_cast<float*>(c + b1 + b2 + b3);
   }
   return b1 + b2 + b3 + b2;
+}
+
+// The partials of all n rows in one window.
+size_t one_window_bytes(int64_t n, int64_t v) {
+  return window_ws_layout(n, head_plan(n, v).splits, nullptr, nullptr);
+}
+
+// The partials of the largest window: the full ones and the last may be planned with
+// different split counts.
+size_t windows_bytes(int64_t n, int64_t v) {
+  const int64_t rows = window_rows(n, v);
+  if (n <= rows) return one_window_bytes(n, v);
+  const size_t a = one_window_bytes(rows, v), b = one_window_bytes(n - (n - 1) / rows * rows, v);
+  return a > b ? a : b;
+}
+
+// Rows per window with ws_bytes of workspace: a window's plan may take more splits, and more
+// partials, than one plan for all rows (4 sizes in 1,000, none at V = 248,320); a workspace
+// with room for the latter only runs all rows as one window.
+int64_t rows_per_window(int64_t n, int64_t v, size_t ws_bytes) {
+  return ws_bytes >= windows_bytes(n, v) ? window_rows(n, v) : n;
 }
 
 struct BwdPlan {
@@ -1445,20 +1502,14 @@ hipError_t launch_head(const HeadParams& p, int grid, hipStream_t st, const char
   return hipGetLastError();
 }
 
+// Pass 1 and the merge of one window; keep: the tile values go to p.z.
 template <typename TT, int FLAGS>
-hipError_t head_forward_typed(HeadParams& p, const HeadPlan& pl, const SlotArgs& a, float* row_stats,
-                              float* metrics, const HeadWs& w, hipStream_t st, int parts) {
-  hipError_t e;
-  if (parts & kHeadStats) {
-    if ((e = launch_head<MODE_STATS, TT, FLAGS>(p, pl.grid, st, "head_stats")) != hipSuccess) return e;
-    const TeacherSpec tl{p.trows, p.nt, p.tlse};
-    if ((e = launch_merge(w.part1, w.zy, p.v, pl.splits, a, row_stats, st, p.tlse ? &tl : nullptr)) != hipSuccess)
-      return e;
-  }
-  if (!(parts & kHeadEmit)) return hipSuccess;
-  p.row_stats = row_stats;
-  if ((e = launch_head<MODE_EMIT, TT, FLAGS>(p, pl.grid, st, "head_emit")) != hipSuccess) return e;
-  return launch_finalize(w.parta, pl.splits, a, row_stats, metrics, st, p.tlse ? w.partk : nullptr);
+hipError_t head_stats_window(const HeadParams& p, const HeadPlan& pl, bool keep, const SlotArgs& a,
+                             const TeacherSpec* ts, float* row_stats, hipStream_t st) {
+  const hipError_t e = keep ? launch_head<MODE_STATS, TT, FLAGS | kKeepZ>(p, pl.grid, st, "head_stats")
+                            : launch_head<MODE_STATS, TT, FLAGS>(p, pl.grid, st, "head_stats");
+  if (e != hipSuccess) return e;
+  return launch_merge(p.part1, p.zy, p.v, pl.splits, a, row_stats, st, p.tlse ? ts : nullptr);
 }
 
 }  // namespace
@@ -1468,47 +1519,145 @@ hipError_t lmhead_forward_prepare() {
   if ((e = head_lds_attr<MODE_STATS, uint16_t, 0>()) || (e = head_lds_attr<MODE_EMIT, uint16_t, 0>()) ||
       (e = head_lds_attr<MODE_STATS, float, 0>()) || (e = head_lds_attr<MODE_EMIT, float, 0>()) ||
       (e = head_lds_attr<MODE_STATS, uint16_t, kTeacherLse>()) || (e = head_lds_attr<MODE_EMIT, uint16_t, kTeacherLse>()) ||
-      (e = head_lds_attr<MODE_STATS, float, kTeacherLse>()) || (e = head_lds_attr<MODE_EMIT, float, kTeacherLse>()))
+      (e = head_lds_attr<MODE_STATS, float, kTeacherLse>()) || (e = head_lds_attr<MODE_EMIT, float, kTeacherLse>()) ||
+      (e = head_lds_attr<MODE_STATS, uint16_t, kKeepZ>()) || (e = head_lds_attr<MODE_STATS, float, kKeepZ>()) ||
+      (e = head_lds_attr<MODE_STATS, uint16_t, kTeacherLse | kKeepZ>()) ||
+      (e = head_lds_attr<MODE_STATS, float, kTeacherLse | kKeepZ>()))
     return e;
   return hipSuccess;
 }
 
+size_t lmhead_required_bytes(int64_t n, int64_t v) { return one_window_bytes(n, v); }
+
+size_t lmhead_min_workspace_bytes(int64_t n, int64_t v) {
+  const size_t a = one_window_bytes(n, v), b = windows_bytes(n, v);
+  return a > b ? a : b;
+}
+
 size_t lmhead_workspace_bytes(int64_t n, int64_t v, int64_t d) {
-  (void)d;
-  return head_ws_layout(n, v, nullptr, nullptr);
+  const size_t least = lmhead_min_workspace_bytes(n, v);
+  if (n == 0 || v == 0 || !keeps_tiles(n, v, d)) return least;
+  const int64_t rows = window_rows(n, v);
+  return align_up(least, 256) + emit_workspace_bytes(n < rows ? n : rows, v);
 }
 
 namespace {
 
-// The fused head's kernel arguments, shared by the forward and the dl re-emission.
-HeadParams head_params(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const void* markov,
-                       int64_t ldm, const MarkovFactors* factors, const void* teacher, int64_t ldt, int64_t d,
-                       int64_t v, const SlotArgs& a, const TeacherSpec* ts, void* dl, int64_t ldd,
-                       const HeadPlan& pl, const HeadWs& w) {
-  HeadParams p = {};
-  p.hidden = static_cast<const uint16_t*>(hidden);
-  p.weight = static_cast<const uint16_t*>(weight);
-  p.markov = static_cast<const uint16_t*>(markov);
-  p.teacher = teacher;
-  p.ldh = ldh; p.ldw = ldw; p.ldm = ldm; p.ldt = ldt;
-  p.n = a.n; p.d = d; p.v = v;
-  p.tt = pl.tt; p.vt = pl.vt; p.splits = pl.splits; p.xa = pl.xa; p.xb = pl.xb;
-  p.labels = a.labels; p.weights = a.weights;
-  p.c_ce = a.c_ce; p.c_kl = a.c_kl; p.inv_acc = a.inv_acc;
-  p.part1 = w.part1; p.zy = w.zy; p.parta = w.parta; p.partk = w.partk;
-  p.dl = static_cast<uint16_t*>(dl); p.ldd = ldd;
-  if (ts) {
-    p.trows = ts->rows; p.nt = ts->nt; p.tlse = ts->lse;
-    // any two gathered rows within 4 GiB of each other (bf16 rows through LDS)
-    p.tdirect = ts->rows && ts->nt > 1 && (ts->nt - 1) * ldt * 2 + 512 > (int64_t)0xffffffffLL;
+// The fused head's operands, and those of one window of rows.
+struct HeadArgs {
+  const uint16_t *hidden, *weight, *markov;
+  const void* teacher;
+  int tdt;
+  int64_t ldh, ldw, ldm, ldt, d, v;
+  const MarkovFactors* factors;
+  TeacherSpec ts;   // nt: the rows of the teacher tensor
+  SlotArgs a;
+  uint16_t* dl;
+  int64_t ldd;
+  float* row_stats;
+};
+
+HeadArgs rows_of(const HeadArgs& x, MarkovFactors* f, int64_t r0, int64_t rows) {
+  HeadArgs w = x;
+  w.a.n = rows;
+  w.hidden += r0 * x.ldh;
+  if (x.markov) w.markov += r0 * x.ldm;
+  w.a.labels += r0;
+  w.a.weights += r0;
+  if (x.ts.rows) {
+    w.ts.rows += r0;
+  } else {
+    w.teacher = static_cast<const char*>(x.teacher) + r0 * x.ldt * (x.tdt == kBF16 ? 2 : 4);
+    if (x.ts.lse) w.ts.lse += r0;
+    w.ts.nt = rows;
   }
-  if (factors) {
-    p.prev = factors->prev;
-    p.w1 = static_cast<const uint16_t*>(factors->w1);
-    p.w2 = static_cast<const uint16_t*>(factors->w2);
-    p.ldw1 = factors->ldw1; p.ldw2 = factors->ldw2; p.r = factors->r;
+  if (x.dl) w.dl += r0 * x.ldd;
+  w.row_stats += r0 * kRowStatWidth;
+  if (x.factors) {
+    *f = *x.factors;
+    f->prev += r0;
+    w.factors = f;
+  }
+  return w;
+}
+
+HeadParams head_params(const HeadArgs& x, const HeadPlan& pl, const HeadWs& w) {
+  HeadParams p = {};
+  p.hidden = x.hidden;
+  p.weight = x.weight;
+  p.markov = x.markov;
+  p.teacher = x.teacher;
+  p.ldh = x.ldh; p.ldw = x.ldw; p.ldm = x.ldm; p.ldt = x.ldt;
+  p.n = x.a.n; p.d = x.d; p.v = x.v;
+  p.tt = pl.tt; p.vt = pl.vt; p.splits = pl.splits; p.xa = pl.xa; p.xb = pl.xb;
+  p.labels = x.a.labels; p.weights = x.a.weights;
+  p.c_ce = x.a.c_ce; p.c_kl = x.a.c_kl; p.inv_acc = x.a.inv_acc;
+  p.part1 = w.part1; p.zy = w.zy; p.parta = w.parta; p.partk = w.partk;
+  p.row_stats = x.row_stats;
+  p.dl = x.dl; p.ldd = x.ldd;
+  p.trows = x.ts.rows; p.nt = x.ts.nt; p.tlse = x.ts.lse;
+  // any two gathered rows within 4 GiB of each other (bf16 rows through LDS)
+  p.tdirect = x.ts.rows && x.ts.nt > 1 && (x.ts.nt - 1) * x.ldt * 2 + 512 > (int64_t)0xffffffffLL;
+  if (x.factors) {
+    p.prev = x.factors->prev;
+    p.w1 = static_cast<const uint16_t*>(x.factors->w1);
+    p.w2 = static_cast<const uint16_t*>(x.factors->w2);
+    p.ldw1 = x.factors->ldw1; p.ldw2 = x.factors->ldw2; p.r = x.factors->r;
   }
   return p;
+}
+
+// Pass 2 through the GEMM again: accept and KL partials to the workspace, dl if it is wanted.
+hipError_t head_emit_window(const HeadParams& p, const HeadPlan& pl, int tdt, hipStream_t st) {
+  if (p.tlse) {
+    if (tdt == kBF16) return launch_head<MODE_EMIT, uint16_t, kTeacherLse>(p, pl.grid, st, "head_emit");
+    return launch_head<MODE_EMIT, float, kTeacherLse>(p, pl.grid, st, "head_emit");
+  }
+  if (tdt == kBF16) return launch_head<MODE_EMIT, uint16_t, 0>(p, pl.grid, st, "head_emit");
+  return launch_head<MODE_EMIT, float, 0>(p, pl.grid, st, "head_emit");
+}
+
+// The passes of one window.
+hipError_t head_window(const HeadArgs& x, int parts, bool keep, void* ws, size_t least, hipStream_t st) {
+  const HeadPlan pl = head_plan(x.a.n, x.v);
+  HeadWs w;
+  window_ws_layout(x.a.n, pl.splits, ws, &w);
+  HeadParams p = head_params(x, pl, w);
+  void* zws = static_cast<char*>(ws) + align_up(least, 256);
+  p.z = keep ? static_cast<float*>(zws) : nullptr;
+  hipError_t e = hipSuccess;
+  if (parts & kHeadStats) {
+    if (p.tlse)
+      e = x.tdt == kBF16 ? head_stats_window<uint16_t, kTeacherLse>(p, pl, keep, x.a, &x.ts, x.row_stats, st)
+                         : head_stats_window<float, kTeacherLse>(p, pl, keep, x.a, &x.ts, x.row_stats, st);
+    else
+      e = x.tdt == kBF16 ? head_stats_window<uint16_t, 0>(p, pl, keep, x.a, &x.ts, x.row_stats, st)
+                         : head_stats_window<float, 0>(p, pl, keep, x.a, &x.ts, x.row_stats, st);
+    if (e != hipSuccess) return e;
+  }
+  if (!(parts & kHeadEmit)) return hipSuccess;
+  if (keep)
+    return emit_from_tiles(zws, x.teacher, x.tdt, x.ldt, x.ts, x.v, x.a, pl.splits, x.dl, x.ldd, x.row_stats, st);
+  if ((e = head_emit_window(p, pl, x.tdt, st)) != hipSuccess) return e;
+  return launch_finalize(w.parta, pl.splits, x.a, x.row_stats, nullptr, st, p.tlse ? w.partk : nullptr);
+}
+
+HeadArgs head_args(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const void* markov, int64_t ldm,
+                   const MarkovFactors* factors, const void* teacher, int tdt, int64_t ldt, int64_t d, int64_t v,
+                   const SlotArgs& a, const TeacherSpec* ts, void* dl, int64_t ldd, float* row_stats) {
+  HeadArgs x = {};
+  x.hidden = static_cast<const uint16_t*>(hidden);
+  x.weight = static_cast<const uint16_t*>(weight);
+  x.markov = static_cast<const uint16_t*>(markov);
+  x.teacher = teacher;
+  x.tdt = tdt;
+  x.ldh = ldh; x.ldw = ldw; x.ldm = ldm; x.ldt = ldt; x.d = d; x.v = v;
+  x.factors = factors;
+  x.ts = ts ? *ts : TeacherSpec{nullptr, a.n, nullptr};
+  x.a = a;
+  x.dl = static_cast<uint16_t*>(dl); x.ldd = ldd;
+  x.row_stats = row_stats;
+  return x;
 }
 
 }  // namespace
@@ -1516,38 +1665,43 @@ HeadParams head_params(const void* hidden, int64_t ldh, const void* weight, int6
 hipError_t lmhead_forward(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const void* markov,
                           int64_t ldm, const MarkovFactors* factors, const void* teacher, int tdt, int64_t ldt,
                           int64_t d, int64_t v, const SlotArgs& a, const TeacherSpec* ts, void* dl, int64_t ldd,
-                          float* row_stats, float* metrics, void* ws, hipStream_t st, int parts) {
+                          float* row_stats, float* metrics, void* ws, size_t ws_bytes, hipStream_t st, int parts) {
   if (a.n == 0) return metrics ? launch_finalize(nullptr, 1, a, row_stats, metrics, st) : hipSuccess;
-  const HeadPlan pl = head_plan(a.n, v);
-  HeadWs w;
-  head_ws_layout(a.n, v, ws, &w);
-  HeadParams p = head_params(hidden, ldh, weight, ldw, markov, ldm, factors, teacher, ldt, d, v, a, ts, dl, ldd, pl, w);
-  if (p.tlse) {
-    if (tdt == kBF16) return head_forward_typed<uint16_t, kTeacherLse>(p, pl, a, row_stats, metrics, w, st, parts);
-    return head_forward_typed<float, kTeacherLse>(p, pl, a, row_stats, metrics, w, st, parts);
+  const HeadArgs x = head_args(hidden, ldh, weight, ldw, markov, ldm, factors, teacher, tdt, ldt, d, v, a, ts, dl,
+                               ldd, row_stats);
+  const size_t least = lmhead_min_workspace_bytes(a.n, v);
+  // pass 2 reads pass 1's values when both run here and the workspace holds them
+  const bool keep = parts == kHeadParts && keeps_tiles(a.n, v, d) && ws_bytes >= lmhead_workspace_bytes(a.n, v, d);
+  const int64_t rows = rows_per_window(a.n, v, ws_bytes);
+  for (int64_t r0 = 0; r0 < a.n; r0 += rows) {
+    MarkovFactors f;
+    const HeadArgs w = rows_of(x, &f, r0, a.n - r0 < rows ? a.n - r0 : rows);
+    if (const hipError_t e = head_window(w, parts, keep, ws, least, st); e != hipSuccess) return e;
   }
-  if (tdt == kBF16) return head_forward_typed<uint16_t, 0>(p, pl, a, row_stats, metrics, w, st, parts);
-  return head_forward_typed<float, 0>(p, pl, a, row_stats, metrics, w, st, parts);
+  // the rows' sums are in row_stats
+  return metrics ? launch_finalize(nullptr, 1, a, row_stats, metrics, st) : hipSuccess;
 }
 
 hipError_t lmhead_emit_dlogits(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const void* markov,
                                int64_t ldm, const MarkovFactors* factors, const void* teacher, int tdt, int64_t ldt,
                                int64_t d, int64_t v, const SlotArgs& a, const TeacherSpec* ts,
-                               const float* row_stats, void* dl, int64_t ldd, void* ws, hipStream_t st) {
+                               const float* row_stats, void* dl, int64_t ldd, void* ws, size_t ws_bytes,
+                               hipStream_t st) {
   if (a.n == 0) return hipSuccess;
-  const HeadPlan pl = head_plan(a.n, v);
-  HeadWs w;
-  head_ws_layout(a.n, v, ws, &w);
-  HeadParams p = head_params(hidden, ldh, weight, ldw, markov, ldm, factors, teacher, ldt, d, v, a, ts, dl, ldd, pl, w);
   // pass 2 alone: the row log-normalisers come from the forward's row_stats, the accept
   // and KL partials it also forms go to the workspace and are not read
-  p.row_stats = row_stats;
-  if (p.tlse) {
-    if (tdt == kBF16) return launch_head<MODE_EMIT, uint16_t, kTeacherLse>(p, pl.grid, st, "head_emit");
-    return launch_head<MODE_EMIT, float, kTeacherLse>(p, pl.grid, st, "head_emit");
+  const HeadArgs x = head_args(hidden, ldh, weight, ldw, markov, ldm, factors, teacher, tdt, ldt, d, v, a, ts, dl,
+                               ldd, const_cast<float*>(row_stats));
+  const int64_t rows = rows_per_window(a.n, v, ws_bytes);
+  for (int64_t r0 = 0; r0 < a.n; r0 += rows) {
+    MarkovFactors f;
+    const HeadArgs xw = rows_of(x, &f, r0, a.n - r0 < rows ? a.n - r0 : rows);
+    const HeadPlan pl = head_plan(xw.a.n, v);
+    HeadWs w;
+    window_ws_layout(xw.a.n, pl.splits, ws, &w);
+    if (const hipError_t e = head_emit_window(head_params(xw, pl, w), pl, tdt, st); e != hipSuccess) return e;
   }
-  if (tdt == kBF16) return launch_head<MODE_EMIT, uint16_t, 0>(p, pl.grid, st, "head_emit");
-  return launch_head<MODE_EMIT, float, 0>(p, pl.grid, st, "head_emit");
+  return hipSuccess;
 }
 
 size_t lmhead_bwd_workspace_bytes(int64_t n, int64_t v, int64_t d, int64_t r, bool norm) {

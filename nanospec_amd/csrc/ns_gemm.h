@@ -181,6 +181,21 @@ __device__ __forceinline__ void vm_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Lanes l and l ^ 32 hold the same token (vocab entries 4 h .. 4 h + 3 of each 8-entry
+// chunk, h = l / 32).  v_permlane32_swap hands every lane both lanes' values in the same
+// order, so a symmetric merge of the two leaves identical bits in both.
+__device__ __forceinline__ void half_pair(float x, float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+
+__device__ __forceinline__ float half_sum(float x) {
+  float a, b;
+  half_pair(x, a, b);
+  return a + b;
+}
+
 // Workgroup -> (tile t, split s) map for a grid of TT x S workgroups, one per CU at a
 // time.  Workgroups are dispatched round-robin over the 8 XCDs, and the workgroups of
 // one XCD share its L2.  With xa > 0 the grid runs in rounds of xa * xb workgroups per

@@ -83,6 +83,12 @@ struct MarkovFactors {
   const void* w2;        // [V, r] bf16, row stride ldw2
   int64_t ldw1, ldw2, r;
 };
+// Workspace of the fused forward: required (partials of all rows in one plan), min (partials by
+// windows of rows, as the full one: the same bits), and the full one, which also holds one
+// window's tile values (kZTile): pass 2 then forms dl from pass 1's values instead of running
+// the GEMM again.
+size_t lmhead_required_bytes(int64_t n, int64_t v);
+size_t lmhead_min_workspace_bytes(int64_t n, int64_t v);
 size_t lmhead_workspace_bytes(int64_t n, int64_t v, int64_t d);
 // Raises the dynamic-LDS limit of every head instantiation lmhead_forward can launch, on the
 // current device (done lazily at launch otherwise; this lets a caller do it before capture).
@@ -94,8 +100,22 @@ constexpr int kHeadStats = 1, kHeadEmit = 2, kHeadParts = kHeadStats | kHeadEmit
 hipError_t lmhead_forward(const void* hidden, int64_t ldh, const void* weight, int64_t ldw,
                           const void* markov, int64_t ldm, const MarkovFactors* factors, const void* teacher,
                           int tdt, int64_t ldt, int64_t d, int64_t v, const SlotArgs& a, const TeacherSpec* ts,
-                          void* dl, int64_t ldd, float* row_stats, float* metrics, void* ws, hipStream_t st,
-                          int parts = kHeadParts);
+                          void* dl, int64_t ldd, float* row_stats, float* metrics, void* ws, size_t ws_bytes,
+                          hipStream_t st, int parts = kHeadParts);
+
+// ---- second pass over kept tile values (emit.hip) ------------------------------
+// One 256 x 256 tile of draft logits (fp32, Markov addend included) as pass 1's accumulators hold
+// it: block (s, wave) = 32 tokens x 128 vocab entries, 16 KB at ((s * 4 + wave) * 16 + k) * 256
+// floats for chunk k = 0..15, 4 floats per lane: token 128 (wave & 1) + 32 s + lane % 32, entries
+// 128 (wave >> 1) + 8 k + 4 (lane / 32) + 0..3.
+constexpr int64_t kZTile = 256 * 256;
+// A window's values (at the workspace's start, [token tiles][vocab tiles] of kZTile) and the
+// partial sums after them.
+size_t emit_workspace_bytes(int64_t n, int64_t v);
+// accept rates (with ts.lse also KL) into row_stats and dl (if not NULL) of a window of a.n rows;
+// `splits`: the vocab splits whose order the row sums follow
+hipError_t emit_from_tiles(void* ws, const void* teacher, int tdt, int64_t ldt, const TeacherSpec& ts, int64_t v,
+                           const SlotArgs& a, int splits, void* dl, int64_t ldd, float* row_stats, hipStream_t st);
 // dst row r = src row map[r] (row_bytes bytes), or zeros where map[r] is outside [0, n_src)
 hipError_t copy_rows(const void* src, int64_t ld_src, int64_t n_src, const int64_t* map, int64_t n_dst,
                      int64_t row_bytes, void* dst, int64_t ld_dst, hipStream_t st);
@@ -106,7 +126,7 @@ hipError_t lmhead_emit_dlogits(const void* hidden, int64_t ldh, const void* weig
                                const void* markov, int64_t ldm, const MarkovFactors* factors, const void* teacher,
                                int tdt, int64_t ldt, int64_t d, int64_t v, const SlotArgs& a,
                                const TeacherSpec* ts, const float* row_stats, void* dl, int64_t ldd, void* ws,
-                               hipStream_t st);
+                               size_t ws_bytes, hipStream_t st);
 // dh workspace; r > 0 adds the Markov column tiles' partials, norm the rms-norm
 // backward's column partials
 size_t lmhead_bwd_workspace_bytes(int64_t n, int64_t v, int64_t d, int64_t r = 0, bool norm = false);

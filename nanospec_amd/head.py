@@ -8,10 +8,10 @@ Reference region (nanospec/train.py:268-312)::
     dl = ops.ce_kl_backward(saved, accumulation_steps)             # train.py:301
     dh = dl @ lm_head.w                               # train.py:302
 
-Here the forward never materialises the [N, V] draft logits: bf16 MFMA tiles of
-hidden . W^T feed an online log-softmax over V for both distributions (pass 1),
-then a second pass recomputes each tile to form the acceptance rate and dl,
-which feeds the dh = dl . W GEMM in the backward.  The metrics keep the
+Here the forward holds at most a 2 GiB window of the [N, V] draft logits: bf16 MFMA tiles of
+hidden . W^T feed an online log-softmax over V for both distributions (pass 1), then a second
+pass forms the acceptance rate and dl from the window's tile values, window by window;
+dl feeds the dh = dl . W GEMM in the backward.  The metrics keep the
 ``LossMetrics`` names; dl is available for the Markov-head backward
 (train.py:303-307).
 """
@@ -251,7 +251,7 @@ def _forward_skipping_masked(o, lm_head_weight, hidden_shape, h, ldh, w, ldw, m,
     inv_acc = 1.0 / accumulation_steps
 
     def part(which, hh, ldhh, mm, ldmm, uu, lduu, yy, ww, rows, dl, row_stats, targs=None):
-        ws = _lib.workspace(_lib.NS_WS_LMHEAD, rows, vocab, d, device)
+        ws = _lib.workspace(_lib.NS_WS_LMHEAD_MIN, rows, vocab, d, device)
         status = lib.ns_lmhead_ce_kl_fwd_part(
             which, _lib.ptr(hh), ldhh, _lib.ptr(w), ldw, _lib.ptr(mm), ldmm, _lib.ptr(uu), _lib.dtype_code(uu), lduu,
             ctypes.byref(targs) if targs is not None else None, _lib.ptr(yy), _lib.ptr(ww), rows, d, vocab,
@@ -304,7 +304,7 @@ def _reemit_dlogits(saved: HeadActivations, accumulation_steps: int) -> torch.Te
     vocab, d = saved.weight.shape
     device = x.h.device
     dl = torch.empty((n, vocab), dtype=torch.bfloat16, device=device)
-    ws = _lib.workspace(_lib.NS_WS_LMHEAD, n, vocab, d, device)
+    ws = _lib.workspace(_lib.NS_WS_LMHEAD_MIN, n, vocab, d, device)
     targs = None
     if x.rows is not None or x.lse is not None:
         targs = _lib.TeacherArgs(_lib.ptr(x.rows), x.u.shape[0] if x.rows is not None else 0, _lib.ptr(x.lse))

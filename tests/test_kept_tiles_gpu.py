@@ -1,0 +1,93 @@
+"""The fused forward's second pass over kept tile values (NS_WS_LMHEAD workspace) against the
+second run of the GEMM it replaces (NS_WS_LMHEAD_MIN): metrics, row statistics and dl are the
+same bits over every form of the teacher and the Markov head, at the edges of token and vocab
+tiles, without dl, and over several windows of rows."""
+
+import ctypes
+
+import pytest
+import torch
+
+from nanospec_amd import _lib, synthetic
+from nanospec_amd.objective import _slot_inputs
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _forward(lib, kind, h, w, u, slots, *, markov=None, factors=None, rows=None, lse=None, want_dl=True):
+    n, d = h.shape
+    v = w.shape[0]
+    wts, y, valid, k = _slot_inputs(slots, n, torch.device(DEV))
+    out = [torch.full((6,), float("nan"), device=DEV), torch.full((n, 8), float("nan"), device=DEV),
+           torch.full((n, v), float("nan"), dtype=torch.bfloat16, device=DEV) if want_dl else None]
+    targs = None
+    if rows is not None or lse is not None:
+        targs = ctypes.byref(_lib.TeacherArgs(_lib.ptr(rows), u.shape[0] if rows is not None else 0, _lib.ptr(lse)))
+    ws = _lib.workspace(kind, n, v, d, torch.device(DEV))
+    ws.fill_(0x7f)
+    tail = (_lib.ptr(u), _lib.dtype_code(u), v, targs, _lib.ptr(y), _lib.ptr(wts), _lib.ptr(valid), n, d, v, k, 0.1,
+            0.9, 0.5, _lib.ptr(out[2]), v, _lib.ptr(out[1]), _lib.ptr(out[0]), _lib.ptr(ws), ws.numel(),
+            _lib.stream(torch.device(DEV)))
+    if factors is None:
+        status = lib.ns_lmhead_ce_kl_fwd(_lib.ptr(h), d, _lib.ptr(w), d, _lib.ptr(markov), v, *tail)
+    else:
+        prev, w1, w2 = factors
+        r = w1.shape[1]
+        status = lib.ns_lmhead_markov_ce_kl_fwd(_lib.ptr(h), d, _lib.ptr(w), d, _lib.ptr(prev), _lib.ptr(w1), r,
+                                                _lib.ptr(w2), r, r, *tail)
+    _lib.check(status, "forward")
+    torch.cuda.synchronize()
+    return out
+
+
+def _assert_same(a, b):
+    for x, y in zip(a, b):
+        if x is not None:   # NaN patterns too
+            assert torch.equal(x.view(torch.int16 if x.dtype == torch.bfloat16 else torch.int32),
+                               y.view(torch.int16 if y.dtype == torch.bfloat16 else torch.int32))
+
+
+@pytest.mark.parametrize("n,d,v", [(8, 64, 8), (40, 64, 264), (264, 128, 2056), (512, 192, 65536 + 136),
+                                   (136, 320, 65536)])
+@pytest.mark.parametrize("form", ["rows", "gathered", "lse", "fp32", "fp32_lse", "factored", "no_dl"])
+def test_kept_values_give_the_same_bits(gpu_lib, n, d, v, form):
+    h, w, markov, u, slots = synthetic.head_inputs(n, d, v, 7000 + n, DEV, ragged=True)
+    slots.target_ids[0, 0] = -100
+    slots.target_ids[0, 1] = v - 1
+    kw = {"markov": markov if n % 16 else None}
+    if form.startswith("fp32"):
+        u = u.float()
+    if form.endswith("lse"):
+        kw["lse"] = torch.logsumexp(u.double(), -1).float()
+    if form == "gathered":
+        u = torch.cat([u, u[: n // 2].flip(0)]).contiguous()
+        kw["rows"] = torch.randint(0, u.shape[0], (n,), device=DEV)
+        kw["rows"][n // 3] = u.shape[0]       # outside: that row's teacher is NaN
+    if form == "factored":
+        prev, w1, w2 = synthetic.markov_factors(n, v, 64, 7100 + n, DEV)
+        prev[n // 2] = v                      # outside: that row's logits are NaN
+        kw = {"factors": (prev, w1, w2)}
+    kw["want_dl"] = form != "no_dl"
+    lib = gpu_lib
+    assert lib.ns_workspace_bytes(_lib.NS_WS_LMHEAD, n, v, d) > lib.ns_workspace_bytes(_lib.NS_WS_LMHEAD_MIN, n, v, d)
+    _assert_same(_forward(lib, _lib.NS_WS_LMHEAD, h, w, u, slots, **kw),
+                 _forward(lib, _lib.NS_WS_LMHEAD_MIN, h, w, u, slots, **kw))
+
+
+def test_several_windows_of_rows(gpu_lib):
+    """V = 2^21 keeps 256 rows' values in a window: 520 rows are three windows.  The same bits as
+    the GEMM run again, and every row's log-normalisers within 1e-5 of fp64's."""
+    n, d, v = 520, 320, 1 << 21
+    h, w, _, u, slots = synthetic.head_inputs(n, d, v, 7300, DEV, ragged=True)
+    a = _forward(gpu_lib, _lib.NS_WS_LMHEAD, h, w, u, slots)
+    b = _forward(gpu_lib, _lib.NS_WS_LMHEAD_MIN, h, w, u, slots)
+    _assert_same(a, b)
+    stats = a[1]
+    for r in (0, 255, 256, 511, 512, 519):
+        z = torch.cat([h[r].double() @ c.double().t() for c in w.split(1 << 18)])
+        lz, lu = torch.logsumexp(z, -1), torch.logsumexp(u[r].double(), -1)
+        assert abs(float(stats[r, 0] - lz)) < 1e-5 * abs(float(lz))
+        assert abs(float(stats[r, 1] - lu)) < 1e-5 * abs(float(lu))
+        p, t = (z - lz).exp(), (u[r].double() - lu).exp()
+        assert float(stats[r, 4]) == pytest.approx(float(torch.minimum(p, t).sum()), rel=1e-4)
