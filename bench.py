@@ -75,7 +75,7 @@ KERNEL_NAMES = [
     (r"head_kernel<0,", "head_stats"),
     (r"head_kernel<1,", "head_emit"),
     (r"head_kernel<2,", "head_linear"),
-    (r"dh_reduce_kernel", "dh_reduce"),
+    (r"sum_partials_kernel<[^,]+, (?:unsigned short|uint16_t)", "dh_reduce"),
     (r"dh_kernel", "dh_gemm"),
     (r"stream_stats_kernel", "stream_stats"),
     (r"stream_group_kernel<[^,]+, [^,]+, true>", "stream_group"),

@@ -1267,36 +1267,66 @@ void dh_kernel(BwdParams p) {
     }
 }
 
-// fp32 sum of split partials [ksplit][N][d] into fp32 out [N][d] (row stride ldo), fixed order.
+// Fixed-order sum of split partials [ksplit][N][d] into out [N][d] (row stride ldo): fp32, or bf16
+// rounded once.  G groups of 256 / G threads: group g adds its
+// contiguous share of the splits in order, then the groups' sums are added in order.  One
+// thread walking 64 splits took 33 us for N = 224, d = 256 (56 workgroups, one load after the
+// other); with 16 groups 7 us.
+template <int G, typename OUT>
 __global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restrict__ part, int ksplit, int64_t n,
-                                                           int64_t d, float* __restrict__ out, int64_t ldo) {
-  const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+                                                           int64_t d, OUT* __restrict__ out, int64_t ldo) {
+  constexpr int Q = 256 / G;   // float4 columns per workgroup
+  const int g = G > 1 ? threadIdx.x / Q : 0, q = threadIdx.x % Q;
+  const int64_t idx = ((int64_t)blockIdx.x * Q + q) * 4;
   const int64_t total = n * d;
+  const int k0 = g * ksplit / G, k1 = (g + 1) * ksplit / G;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (idx < total && k0 < k1) {
+    s = *reinterpret_cast<const float4*>(part + (int64_t)k0 * total + idx);
+#pragma unroll 4
+    for (int k = k0 + 1; k < k1; ++k) {
+      const float4 x = *reinterpret_cast<const float4*>(part + (int64_t)k * total + idx);
+      s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
+    }
+  }
+  if constexpr (G > 1) {
+    __shared__ float4 sh[G][Q];
+    sh[g][q] = s;
+    __syncthreads();
+    if (g > 0) return;
+#pragma unroll
+    for (int j = 1; j < G; ++j) {
+      const float4 x = sh[j][q];
+      s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
+    }
+  }
   if (idx >= total) return;
   const int64_t row = idx / d, col = idx % d;
-  float4 s = *reinterpret_cast<const float4*>(part + idx);
-  for (int k = 1; k < ksplit; ++k) {
-    const float4 x = *reinterpret_cast<const float4*>(part + (int64_t)k * total + idx);
-    s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
+  if constexpr (sizeof(OUT) == 4) {
+    *reinterpret_cast<float4*>(out + row * ldo + col) = s;
+  } else {
+    uint2 o;
+    o.x = pack_bf16x2(s.x, s.y);
+    o.y = pack_bf16x2(s.z, s.w);
+    *reinterpret_cast<uint2*>(out + row * ldo + col) = o;
   }
-  *reinterpret_cast<float4*>(out + row * ldo + col) = s;
 }
 
-__global__ __launch_bounds__(256) void dh_reduce_kernel(const float* __restrict__ part, int ksplit, int64_t n,
-                                                        int64_t d, uint16_t* __restrict__ dh, int64_t lddh) {
-  const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  const int64_t total = n * d;
-  if (idx >= total) return;
-  const int64_t row = idx / d, col = idx % d;
-  float4 s = *reinterpret_cast<const float4*>(part + idx);
-  for (int k = 1; k < ksplit; ++k) {
-    const float4 x = *reinterpret_cast<const float4*>(part + (int64_t)k * total + idx);
-    s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
-  }
-  uint2 o;
-  o.x = pack_bf16x2(s.x, s.y);
-  o.y = pack_bf16x2(s.z, s.w);
-  *reinterpret_cast<uint2*>(dh + row * lddh + col) = o;
+template <typename OUT>
+hipError_t launch_sum_partials(const float* part, int ksplit, int64_t n, int64_t d, OUT* out, int64_t ldo,
+                               hipStream_t st) {
+  const int64_t quads = (n * d + 3) / 4;
+  const int groups = split_groups(ksplit);
+  if (groups == 1)
+    hipLaunchKernelGGL((sum_partials_kernel<1, OUT>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, part,
+                       ksplit, n, d, out, ldo);
+  else if (groups == 4)
+    hipLaunchKernelGGL((sum_partials_kernel<4, OUT>), dim3((unsigned)((quads + 63) / 64)), dim3(256), 0, st, part,
+                       ksplit, n, d, out, ldo);
+  else
+    hipLaunchKernelGGL((sum_partials_kernel<16, OUT>), dim3((unsigned)((quads + 15) / 16)), dim3(256), 0, st, part,
+                       ksplit, n, d, out, ldo);
+  return hipGetLastError();
 }
 
 // CUs of the current device (cached per device id below 64; 256 when the query fails, as
@@ -1412,6 +1442,16 @@ struct BwdPlan {
   int xa, xb;        // XCD block (dh_kernel's tile order), 0 = unblocked
 };
 
+// K splits of the dh GEMM: of the counts that fill 1, 2, .. kMaxRounds rounds of the CUs, the one
+// of least cost in units of a K entry of one 256 x 256 tile (24 ns: 0.77 us a 32-K stage):
+// rounds x (a workgroup's share of K + kTileCost for its first fills and its partial tile's
+// store, about 15 us) + the partials' sum (4 bytes per entry and split at 4.5 TB/s).  (ceil of
+// four rounds, at most 16 splits, gave N = 1001, d = 5120, V = 248,320 13 splits, 4.06 rounds:
+// 2.34 ms, with 16 1.89; N = 224 16 splits, 1.25 rounds: 0.77 ms, with 12 0.64; N = 64, d = 256
+// 16 workgroups.)
+constexpr int kMaxRounds = 6;
+constexpr double kTileCost = 640, kPartialCost = 3.7e-5;
+
 BwdPlan bwd_plan(int64_t n, int64_t v, int64_t d, int64_t r = 0) {
   BwdPlan pl;
   pl.mt = (int)((n + BM - 1) / BM);
@@ -1420,10 +1460,21 @@ BwdPlan bwd_plan(int64_t n, int64_t v, int64_t d, int64_t r = 0) {
   pl.kt_total = (int)((v + BK - 1) / BK);
   const int tiles = pl.mt * pl.ct;
   const int cus = device_cus();
-  int ks = tiles > 0 ? (4 * cus + tiles - 1) / tiles : 1;   // no tiles: nothing launches
-  if (ks < 1) ks = 1;
-  if (ks > 16) ks = 16;
-  if (ks > pl.kt_total) ks = pl.kt_total;
+  int ks = 1;   // no tiles: nothing launches
+  if (tiles > 0) {
+    double best = 0;
+    for (int j = 1; j <= kMaxRounds; ++j) {
+      int c = (int)((int64_t)j * cus / tiles);
+      if (c < 1) c = 1;
+      if (c > pl.kt_total) c = pl.kt_total;
+      const double cost = ((int64_t)tiles * c + cus - 1) / cus * ((double)v / c + kTileCost) +
+                          (double)c * n * d * kPartialCost;
+      if (j == 1 || cost < best) {
+        best = cost;
+        ks = c;
+      }
+    }
+  }
   pl.ksplit = ks;
   pl.grid_main = tiles * ks;
   // Markov tiles run after the dh tiles as one extra round: enough K splits to give
@@ -1759,19 +1810,13 @@ hipError_t lmhead_backward_ext(const void* dl, int64_t ldd, const void* weight, 
     hipError_t e = rms_norm_backward_rows(p.part, pl.ksplit, nullptr, 0, *norm, dh, lddh, n, d, norm_ws, st);
     if (e != hipSuccess) return e;
   } else {
-    const int64_t quads = (n * d + 3) / 4;
     NS_TIMED("dh_reduce", st);
-    hipLaunchKernelGGL(dh_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, p.part, pl.ksplit,
-                       n, d, static_cast<uint16_t*>(dh), lddh);
-    hipError_t e = hipGetLastError();
+    const hipError_t e = launch_sum_partials(p.part, pl.ksplit, n, d, static_cast<uint16_t*>(dh), lddh, st);
     if (e != hipSuccess) return e;
   }
   if (r > 0) {
-    const int64_t quads = (n * r + 3) / 4;
     NS_TIMED("dprev_reduce", st);
-    hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, p.part2,
-                       pl.ksplit2, n, r, dprev, r);
-    return hipGetLastError();
+    return launch_sum_partials(p.part2, pl.ksplit2, n, r, dprev, r, st);
   }
   return hipSuccess;
 }

@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kThreads) void rms_fwd_kernel(const uint16_t* __res
 }
 
 // rms_norm backward over a block of `rows` rows per workgroup.  dy comes either from
-// split-K partials part[ksplit][N][d] (fp32, summed in split order and rounded to bf16,
+// split-K partials part[ksplit][N][d] (fp32, summed in a fixed order and rounded to bf16,
 // which is the reference's bf16 dh) or from a bf16 tensor.  Writes dx (bf16) and this
 // block's column sums of bf16(dy * normalized) into wpart[block][d] (fp32).
 template <bool FROM_PARTS>
@@ -95,12 +95,21 @@ __global__ __launch_bounds__(kThreads) void rms_bwd_kernel(const float* __restri
       if (c < d) {
         float dy[8];
         if (FROM_PARTS) {
-          load8(part + row * d + c, dy);
-          for (int k = 1; k < ksplit; ++k) {
-            float t[8];
-            load8(part + ((int64_t)k * n + row) * d + c, t);
+          // the order of sum_partials_kernel: groups of splits, then their sums
+          const int groups = split_groups(ksplit);
+          for (int g = 0; g < groups; ++g) {
+            const int k0 = g * ksplit / groups, k1 = (g + 1) * ksplit / groups;
+            float s[8];
+            load8(part + ((int64_t)k0 * n + row) * d + c, s);
+#pragma unroll 4
+            for (int k = k0 + 1; k < k1; ++k) {
+              float t[8];
+              load8(part + ((int64_t)k * n + row) * d + c, t);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) dy[e] += t[e];
+              for (int e = 0; e < 8; ++e) s[e] += t[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dy[e] = g == 0 ? s[e] : dy[e] + s[e];
           }
 #pragma unroll
           for (int e = 0; e < 8; ++e) dy[e] = bf16r(dy[e]);

@@ -178,6 +178,10 @@ hipError_t pooled_tail(const float* metrics, int64_t count, int64_t world_size, 
 // grad[0..n) *= *factor in place (bf16 or fp32)
 hipError_t scale_gradient(void* grad, int dtype, int64_t n, const float* factor, hipStream_t st);
 
+// Groups of splits that the sums of split-K partials are formed in: each group's contiguous share
+// (group g: splits [g * ksplit / G, (g + 1) * ksplit / G)) in order, then the groups in order.
+__host__ __device__ inline int split_groups(int ksplit) { return ksplit <= 8 ? 1 : ksplit <= 24 ? 4 : 16; }
+
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // Raises a kernel's dynamic-LDS limit to `bytes` on the current device.  The attribute
