@@ -150,39 +150,56 @@ __global__ __launch_bounds__(kThreads) void rms_bwd_kernel(const float* __restri
   }
 }
 
-// weight_grad[c] = bf16(sum over blocks of wpart[b][c]): 1024 threads per 256 columns,
-// 16 strided groups of blocks each summed in order, then the groups in order.
+// weight_grad[c] = bf16(sum over blocks of wpart[b][c]): 1024 threads per kWgCols columns, the
+// blocks in kWgGroups strided groups each summed in order, then the groups in eight runs of
+// sixteen, then the runs.  32 columns (a 128-byte line per group and step) rather than 256: at
+// N = 1792, d = 5120 20 workgroups of 16 groups took 38 us, 160 of 128 groups 7 us.
+constexpr int kWgCols = 32, kWgQuads = kWgCols / 4, kWgGroups = 1024 / kWgQuads;
 __global__ __launch_bounds__(1024) void rms_wgrad_kernel(const float* __restrict__ wpart, int64_t nblk, int64_t d,
                                                          uint16_t* __restrict__ wgrad) {
-  __shared__ float4 acc[16][64];
-  const int q = threadIdx.x & 63, grp = threadIdx.x >> 6;
-  const int64_t c = (int64_t)blockIdx.x * 256 + q * 4;
+  __shared__ float4 acc[kWgGroups][kWgQuads];
+  __shared__ float4 run[8][kWgQuads];
+  const int q = threadIdx.x % kWgQuads, grp = threadIdx.x / kWgQuads;
+  const int64_t c = (int64_t)blockIdx.x * kWgCols + q * 4;
   float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
   if (c < d) {
-    for (int64_t b = grp; b < nblk; b += 16) {
+#pragma unroll 4
+    for (int64_t b = grp; b < nblk; b += kWgGroups) {
       const float4 t = *reinterpret_cast<const float4*>(wpart + b * d + c);
       s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
     }
   }
   acc[grp][q] = s;
   __syncthreads();
-  if (grp == 0 && c < d) {
-    float4 t = acc[0][q];
-    for (int g = 1; g < 16; ++g) {
-      t.x += acc[g][q].x; t.y += acc[g][q].y; t.z += acc[g][q].z; t.w += acc[g][q].w;
-    }
-    uint2 o;
-    o.x = pack_bf16x2(t.x, t.y);
-    o.y = pack_bf16x2(t.z, t.w);
-    *reinterpret_cast<uint2*>(wgrad + c) = o;
+  if (grp >= 8) return;   // the first wave goes on
+  s = acc[grp * (kWgGroups / 8)][q];
+#pragma unroll
+  for (int g = 1; g < kWgGroups / 8; ++g) {
+    const float4 t = acc[grp * (kWgGroups / 8) + g][q];
+    s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
   }
+  run[grp][q] = s;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (grp > 0 || c >= d) return;
+#pragma unroll
+  for (int g = 1; g < 8; ++g) {
+    const float4 t = run[g][q];
+    s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
+  }
+  uint2 o;
+  o.x = pack_bf16x2(s.x, s.y);
+  o.y = pack_bf16x2(s.z, s.w);
+  *reinterpret_cast<uint2*>(wgrad + c) = o;
 }
 
 }  // namespace
 
 int norm_rows_per_block(int64_t n) {
-  // enough workgroups to cover the CUs several times over, few enough column partials
-  return n >= 8192 ? 16 : (n >= 2048 ? 4 : 1);
+  // enough workgroups to cover the CUs several times over, few enough column partials (N = 1792,
+  // d = 5120: 25 + 10 us for the pass and the partials' sum with one row, 22 + 7 with two, 21 + 6
+  // with four, which leave N = 1024 one workgroup a CU)
+  return n >= 8192 ? 16 : n >= 2048 ? 4 : n >= 1024 ? 2 : 1;
 }
 
 size_t norm_bwd_workspace_bytes(int64_t n, int64_t d) {
@@ -218,7 +235,7 @@ hipError_t rms_norm_backward_rows(const float* part, int ksplit, const void* dy,
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   NS_TIMED("rms_norm_wgrad", st);
-  hipLaunchKernelGGL(rms_wgrad_kernel, dim3((unsigned)((d + 255) / 256)), dim3(1024), 0, st, wpart, nblk, d,
+  hipLaunchKernelGGL(rms_wgrad_kernel, dim3((unsigned)((d + kWgCols - 1) / kWgCols)), dim3(1024), 0, st, wpart, nblk, d,
                      nb.wgrad);
   return hipGetLastError();
 }
