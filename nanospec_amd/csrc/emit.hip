@@ -226,9 +226,10 @@ void emit_tiles_kernel(EmitParams p) {
 
 // Row sums of the half tiles' partials in the order head_kernel<EMIT> and row_parts_kernel add
 // them: each vocab half's tiles of a split in tile order, the halves, then the splits in order.
-// 16 rows x 16 split lanes per workgroup.
-constexpr int kSumRows = 16;
-template <bool LSE>
+// kSumRows rows x 256 / kSumRows split lanes per workgroup: 16 rows, or 4 past 48 splits (few
+// rows: with 16, N = 224, 256 splits took 30 us for 15, N = 1001, 64 splits 23 for 15; N = 2048,
+// 32 splits 15 us for 24 the other way round).
+template <bool LSE, int kSumRows>
 __global__ __launch_bounds__(256) void emit_rows_kernel(const float* __restrict__ asum, const float* __restrict__ ksum,
                                                         int64_t rows, int vt, int splits, int64_t n,
                                                         float* __restrict__ row_stats) {
@@ -273,9 +274,15 @@ hipError_t launch(const EmitParams& p, int splits, float* row_stats, hipStream_t
     if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
   NS_TIMED("row_parts", st);
-  hipLaunchKernelGGL(emit_rows_kernel<LSE>, dim3((unsigned)((p.n + kSumRows - 1) / kSumRows)), dim3(256),
-                     (size_t)splits * kSumRows * sizeof(float) * (LSE ? 2 : 1), st, p.asum, p.ksum, p.rows, p.vt,
-                     splits, p.n, row_stats);
+  const int rows = splits > 48 ? 4 : 16;
+  const dim3 grid((unsigned)((p.n + rows - 1) / rows));
+  const size_t lds = (size_t)splits * rows * sizeof(float) * (LSE ? 2 : 1);
+  if (rows == 4)
+    hipLaunchKernelGGL((emit_rows_kernel<LSE, 4>), grid, dim3(256), lds, st, p.asum, p.ksum, p.rows, p.vt, splits, p.n,
+                       row_stats);
+  else
+    hipLaunchKernelGGL((emit_rows_kernel<LSE, 16>), grid, dim3(256), lds, st, p.asum, p.ksum, p.rows, p.vt, splits,
+                       p.n, row_stats);
   return hipGetLastError();
 }
 

@@ -223,12 +223,15 @@ constexpr int kSeg = 64;           // sorted positions per piece segment (one wa
 
 int64_t sort_padded(int64_t n) { return (n + kSortChunk - 1) / kSortChunk * kSortChunk; }
 
-// Build the keys of one chunk and bitonic-sort it in LDS (ascending).
+// Build the keys of one chunk and bitonic-sort it in LDS (ascending).  `chunk`: kSortChunk, or
+// for n below it the power of two that holds the n keys (N = 224: 256 keys, 36 steps instead of
+// 78 over 4096).
 __global__ __launch_bounds__(kSortThreads) void markov_sort_chunks_kernel(const int64_t* __restrict__ prev, int64_t n,
-                                                                         int64_t v, uint64_t* __restrict__ out) {
+                                                                         int64_t v, int chunk,
+                                                                         uint64_t* __restrict__ out) {
   __shared__ uint64_t sk[kSortChunk];
-  const int64_t base = (int64_t)blockIdx.x * kSortChunk;
-  for (int i = threadIdx.x; i < kSortChunk; i += kSortThreads) {
+  const int64_t base = (int64_t)blockIdx.x * chunk;
+  for (int i = threadIdx.x; i < chunk; i += kSortThreads) {
     const int64_t t = base + i;
     uint64_t k;
     if (t < n) {
@@ -241,9 +244,9 @@ __global__ __launch_bounds__(kSortThreads) void markov_sort_chunks_kernel(const 
     sk[i] = k;
   }
   __syncthreads();
-  for (int size = 2; size <= kSortChunk; size <<= 1) {
+  for (int size = 2; size <= chunk; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int q = threadIdx.x; q < kSortChunk / 2; q += kSortThreads) {
+      for (int q = threadIdx.x; q < chunk / 2; q += kSortThreads) {
         // pair q: element i with bit `stride` clear and its partner i + stride
         const int i = (q / stride) * 2 * stride + (q % stride);
         const int j = i + stride;
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(kSortThreads) void markov_sort_chunks_kernel(const 
       __syncthreads();
     }
   }
-  for (int i = threadIdx.x; i < kSortChunk; i += kSortThreads) out[base + i] = sk[i];
+  for (int i = threadIdx.x; i < chunk; i += kSortThreads) out[base + i] = sk[i];
 }
 
 // Merge sorted runs of length len pairwise (runs 2m and 2m + 1) from src into dst, n_pad
@@ -299,17 +302,28 @@ __global__ __launch_bounds__(256) void markov_pieces_kernel(const uint64_t* __re
     const bool act = c < r;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     int start = 0;
-    for (int j = 0; j < cnt; ++j) {
-      const int row = __shfl(row_m, j), tok = __shfl(tok_m, j);
-      const int next = __shfl(row_m, j + 1 < cnt ? j + 1 : j);
-      if (act) {
-        const float4 x = *reinterpret_cast<const float4*>(dprev + (int64_t)tok * r + c);
-        acc.x += x.x; acc.y += x.y; acc.z += x.z; acc.w += x.w;
+    // eight rows loaded before the first is added (one after the other, a segment's 64 round
+    // trips took most of 55 us at N = 224)
+    for (int jb = 0; jb < cnt; jb += 8) {
+      float4 x[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int tok = __builtin_amdgcn_readlane(tok_m, jb + q < cnt ? jb + q : cnt - 1);
+        x[q] = *reinterpret_cast<const float4*>(dprev + (int64_t)tok * r + (act ? c : 0));
       }
-      if (j + 1 == cnt || next != row) {
-        if (act && (uint32_t)row < (uint64_t)v) *reinterpret_cast<float4*>(piece + (s0 + start) * r + c) = acc;
-        acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        start = j + 1;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int j = jb + q;
+        if (j < cnt) {
+          const int row = __builtin_amdgcn_readlane(row_m, j);
+          const int next = __builtin_amdgcn_readlane(row_m, j + 1 < cnt ? j + 1 : j);
+          acc.x += x[q].x; acc.y += x[q].y; acc.z += x[q].z; acc.w += x[q].w;
+          if (j + 1 == cnt || next != row) {
+            if (act && (uint32_t)row < (uint64_t)v) *reinterpret_cast<float4*>(piece + (s0 + start) * r + c) = acc;
+            acc = make_float4(0.f, 0.f, 0.f, 0.f);
+            start = j + 1;
+          }
+        }
       }
     }
   }
@@ -406,8 +420,10 @@ hipError_t markov_backward(const void* dl, int64_t ldd, const void* weight, int6
   {
     NS_TIMED("markov_sort", st);
     const int64_t n_pad = sort_padded(n);
+    int chunk = kSortChunk;
+    while (chunk > 64 && chunk / 2 >= n) chunk /= 2;
     hipLaunchKernelGGL(markov_sort_chunks_kernel, dim3((unsigned)(n_pad / kSortChunk)), dim3(kSortThreads), 0, st,
-                       f.prev, n, v, w.keys_a);
+                       f.prev, n, v, chunk, w.keys_a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     for (int64_t len = kSortChunk; len < n_pad; len *= 2) {
       hipLaunchKernelGGL(markov_merge_kernel, dim3((unsigned)((n_pad + 255) / 256)), dim3(256), 0, st, w.keys_a,
