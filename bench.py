@@ -103,6 +103,7 @@ KERNEL_NAMES = [
     (r"fp8_quant_kernel", "fp8_quant"),
     (r"fp8_head_kernel", "fp8_head_gemm"),
     (r"copy_rows_kernel", "copy_rows"),
+    (r"kept_rows_kernel", "kept_rows"),
     (r"prepare_kernel", "prepare_slots"),
 ]
 # profiles/<prefix>_traffic.md and <prefix>_kernel_stats.md: named for the kernels and workload
@@ -601,16 +602,15 @@ def workload_head(device, args, which):
     kernel_flops = {"head_stats": gemm, "dh_gemm": gemm}
     rows2 = n
     if skip:
-        # pass 2 and the dh GEMM run on the rows whose dl is not all zero: here the supervised
-        # ones (every row's statistics are finite); their executed work, not N's
+        # dl and the dh GEMM run on the supervised rows; their executed work, not N's
         rows2 = int(((slots.valid.reshape(-1) != 0) | (slots.weights.reshape(-1) != 0)).sum())
-        kernel_flops = {"head_stats": gemm, "head_emit": 2.0 * rows2 * v * d, "dh_gemm": 2.0 * rows2 * v * d}
+        kernel_flops = {"head_stats": gemm, "dh_gemm": 2.0 * rows2 * v * d}
     kernel_fp8_flops = {"fp8_head_gemm": gemm} if fp8 is not None else {}
     # byte streams (for the per-kernel GB/s report): pass 1 reads Markov + teacher and writes
     # its fp32 values, pass 2 reads them and the teacher and writes dl; the dh GEMM reads dl
     kernel_bytes = {"head_stats": 8 * n * v, "head_emit": 8 * n * v, "dh_gemm": 2 * n * v}
-    if skip:   # pass 1 keeps nothing, pass 2 runs the GEMM on its rows
-        kernel_bytes = {"head_stats": 4 * n * v, "head_emit": 6 * rows2 * v, "dh_gemm": 2 * rows2 * v}
+    if skip:   # pass 2 reads every row's values, the supervised rows' teacher
+        kernel_bytes = {"head_stats": 8 * n * v, "head_emit": 4 * n * v + 4 * rows2 * v, "dh_gemm": 2 * rows2 * v}
 
     def cpu_baseline(rows):
         import numpy as np
@@ -661,7 +661,7 @@ def workload_head(device, args, which):
                           f"ce_kl_loss, ce_kl_backward, dh GEMM; d={d}, V={v}; {threads} threads", extra)
 
     name = {"c2": "C2 full fused", "c3": "C3 long-batch", "c4": "C4 FP8 teacher head + full fused",
-            "c3s": "C3 long-batch, pass 2 and dhidden on the rows with a nonzero dl only"}[which]
+            "c3s": "C3 long-batch, dl and dhidden for the supervised rows only"}[which]
     config = {"workload": f"{name}: LM-head GEMM + Markov addend + CE+KL+accept fwd, dl + dhidden bwd",
               "N": n, "d": d, "V": v, "K": 8, "gamma": gamma, "global_batch": n, "seq_len": None,
               "parallelism": "single GPU"}
@@ -680,7 +680,7 @@ def workload_head(device, args, which):
             out["fp8"] = fp8_ceilings(fp8)
         return out
 
-    executed = gemm + 4.0 * rows2 * v * d if skip else None   # pass 1 on N rows, pass 2 and dh on rows2
+    executed = gemm + 2.0 * rows2 * v * d if skip else None   # pass 1 on N rows, dh on rows2
     return dict(step=step, n=n, per_slot_bytes=None, per_slot_flops=4.0 * v * d, kernel_bytes=kernel_bytes,
                 stream_kernels=("head_emit",), executed_flops_per_step=executed,
                 kernel_flops=kernel_flops, kernel_fp8_flops=kernel_fp8_flops, cpu_baseline=cpu_baseline,

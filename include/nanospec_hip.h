@@ -69,6 +69,7 @@ extern "C" {
 #define NS_WS_RMS_NORM_BWD 4     /* ns_rms_norm_bwd (v ignored) */
 #define NS_WS_LMHEAD_NORM_BWD 5  /* ns_lmhead_norm_bwd */
 #define NS_WS_TEACHER_LOGITS 6   /* ns_lmhead_teacher_logits with lse (d ignored) */
+#define NS_WS_LMHEAD_ROWS 8      /* ns_lmhead_ce_kl_fwd_rows (d ignored) */
 #define NS_WS_LMHEAD_MIN 7       /* what every fused-head entry accepts (d ignored): pass 2 runs the GEMM again */
 
 typedef struct ihipStream_t* ns_stream_t; /* == hipStream_t */
@@ -143,11 +144,9 @@ int ns_lmhead_ce_kl_fwd(const void* hidden, int64_t ldh, const void* weight, int
                         float inv_acc, void* dl, int64_t ldd, float* row_stats, float* metrics, void* workspace,
                         size_t workspace_bytes, ns_stream_t stream);
 
-/* The fused forward in two parts, for a caller that runs pass 2 on a subset of its rows:
- * head.lm_head_ce_kl_loss(skip_masked_rows=True) runs pass 1 on every row, then pass 2 and
- * the dh GEMM only on the rows whose dl is not all zero (supervised rows, and unsupervised
- * rows whose log-normalisers are not finite), gathered with ns_copy_rows.  No counterpart in
- * the reference: objective.py:49-67 in steps.
+/* The fused forward in two parts, for a caller that runs pass 2 on a subset of its rows,
+ * gathered with ns_copy_rows (ns_lmhead_ce_kl_fwd_rows does so without a second GEMM).  No
+ * counterpart in the reference: objective.py:49-67 in steps.
  *   NS_PART_STATS: pass 1 and the merge; writes row_stats' lse_z, lse_u, ce, kl and z_label
  *                  (dl is ignored).
  *   NS_PART_EMIT:  pass 2 from row_stats' log-normalisers; writes dl (when not NULL) and the
@@ -169,9 +168,30 @@ int ns_lmhead_ce_kl_fwd_part(int part, const void* hidden, int64_t ldh, const vo
 int ns_objective_metrics(const float* row_stats, const float* weights, const uint8_t* valid, int64_t n, int64_t k,
                          float c_ce, float c_kl, float* metrics, ns_stream_t stream);
 
-/* dst row r = src row map[r] (row_bytes bytes each) for r < n_dst, and zeros where map[r] is
- * outside [0, n_src): the gather of the rows ns_lmhead_ce_kl_fwd_part runs pass 2 on, and the
- * scatter of their dl and dh back among zero rows.  Pitches in bytes; row_bytes and pitches
+/* ns_lmhead_ce_kl_fwd with dl formed for some rows only: row t's dl goes to row dl_rows[t] of
+ * dl [n_dl, V]; rows whose dl_rows is outside [0, n_dl) have none.  Their accept rate is 0, or
+ * NaN when a log-normaliser is not finite (their dl would be 0 * NaN), and dl_rows is set to -1,
+ * or NS_ROW_NAN, accordingly, for ns_copy_rows to scatter dl and dh among zero (NaN) rows.  The
+ * rows left out must have valid 0 and weight 0.  Dense or no Markov addend; teacher_args as in
+ * ns_lmhead_ce_kl_fwd without lse.  Workspace NS_WS_LMHEAD_ROWS.  No counterpart in the reference. */
+#define NS_ROW_NAN INT64_MIN
+int ns_lmhead_ce_kl_fwd_rows(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const void* markov,
+                             int64_t ldm, const void* teacher, int t_dtype, int64_t ldt,
+                             const ns_teacher_args* teacher_args, const int64_t* labels, const float* weights,
+                             const uint8_t* valid, int64_t n, int64_t d, int64_t v, int64_t k, float c_ce,
+                             float c_kl, float inv_acc, void* dl, int64_t ldd, int64_t* dl_rows, int64_t n_dl,
+                             float* row_stats, float* metrics, void* workspace, size_t workspace_bytes,
+                             ns_stream_t stream);
+
+/* index[r] = the place of row r among the supervised rows (valid[r] != 0 or weights[r] != 0), in
+ * order, or -1; count[0] = their number (device memory). */
+int ns_kept_rows(const float* weights, const uint8_t* valid, int64_t n, int64_t* index, int64_t* count,
+                 ns_stream_t stream);
+
+/* dst row r = src row map[r] (row_bytes bytes each) for r < n_dst, zeros where map[r] is
+ * outside [0, n_src), bytes of 0xFF where it is NS_ROW_NAN: the gather of the rows
+ * ns_lmhead_ce_kl_fwd_part runs pass 2 on, and the scatter of dl and dh back among zero rows.
+ * Pitches in bytes; row_bytes and pitches
  * multiples of 4 (16-byte accesses when all are multiples of 16).  No counterpart in the
  * reference. */
 int ns_copy_rows(const void* src, int64_t ld_src, int64_t n_src, const int64_t* map, int64_t n_dst, int64_t row_bytes,

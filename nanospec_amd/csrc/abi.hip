@@ -97,6 +97,8 @@ size_t ns_workspace_bytes(int kind, int64_t n, int64_t v, int64_t d) {
       return ns::lmhead_linear_lse_workspace_bytes(n, v);
     case NS_WS_LMHEAD_MIN:
       return ns::lmhead_min_workspace_bytes(n, v);
+    case NS_WS_LMHEAD_ROWS:
+      return n > 0 && v > 0 ? ns::lmhead_rows_workspace_bytes(n, v) : 0;
     default:
       return 0;
   }
@@ -263,6 +265,41 @@ int ns_lmhead_ce_kl_fwd_part(int part, const void* hidden, int64_t ldh, const vo
                                        reinterpret_cast<hipStream_t>(stream),
                                        part == NS_PART_STATS ? ns::kHeadStats : ns::kHeadEmit),
                     "ns_lmhead_ce_kl_fwd_part");
+}
+
+int ns_lmhead_ce_kl_fwd_rows(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const void* markov,
+                             int64_t ldm, const void* teacher, int t_dtype, int64_t ldt,
+                             const ns_teacher_args* teacher_args, const int64_t* labels, const float* weights,
+                             const uint8_t* valid, int64_t n, int64_t d, int64_t v, int64_t k, float c_ce,
+                             float c_kl, float inv_acc, void* dl, int64_t ldd, int64_t* dl_rows, int64_t n_dl,
+                             float* row_stats, float* metrics, void* workspace, size_t workspace_bytes,
+                             ns_stream_t stream) {
+  if (n_dl < 0 || n_dl > n || n >= (int64_t(1) << 31) || (n > 0 && !dl_rows))
+    return fail(NS_EINVAL, "dl_rows must be non-NULL and n_dl in [0, n], n below 2^31");
+  if (teacher_args && teacher_args->lse) return fail(NS_EINVAL, "dl by rows takes no teacher log-normalisers");
+  if (n_dl > 0 && !dl) return fail(NS_ENULL, "dl is NULL");
+  int64_t nt = 0;
+  int rc = check_head_inputs(hidden, ldh, weight, ldw, markov, ldm, nullptr, teacher, t_dtype, ldt, teacher_args,
+                             labels, weights, valid, n, d, v, k, n_dl > 0 ? dl : nullptr, ldd, row_stats, metrics,
+                             workspace, workspace_bytes, kCheckForward, &nt);
+  if (rc) return rc;
+  const size_t need = n > 0 ? ns::lmhead_rows_workspace_bytes(n, v) : 0;
+  if (workspace_bytes < need)
+    return fail(NS_EWORKSPACE, "workspace of %zu bytes required (got %zu)", need, workspace_bytes);
+  ns::SlotArgs a{labels, weights, valid, n, k, c_ce, c_kl, inv_acc};
+  const ns::TeacherSpec ts{teacher_args ? teacher_args->rows : nullptr, nt, nullptr};
+  return hip_status(ns::lmhead_forward(hidden, ldh, weight, ldw, markov, ldm, nullptr, teacher, t_dtype, ldt, d, v, a,
+                                       &ts, n_dl > 0 ? dl : nullptr, ldd, row_stats, metrics, workspace,
+                                       workspace_bytes, reinterpret_cast<hipStream_t>(stream), ns::kHeadParts,
+                                       dl_rows, n_dl),
+                    "ns_lmhead_ce_kl_fwd_rows");
+}
+
+int ns_kept_rows(const float* weights, const uint8_t* valid, int64_t n, int64_t* index, int64_t* count,
+                 ns_stream_t stream) {
+  if (n < 0) return fail(NS_EINVAL, "n must be >= 0 (got %lld)", (long long)n);
+  if (!count || (n > 0 && (!weights || !valid || !index))) return fail(NS_ENULL, "weights, valid, index and count must be non-NULL");
+  return hip_status(ns::kept_rows(weights, valid, n, index, count, reinterpret_cast<hipStream_t>(stream)), "ns_kept_rows");
 }
 
 int ns_objective_metrics(const float* row_stats, const float* weights, const uint8_t* valid, int64_t n, int64_t k,

@@ -29,6 +29,10 @@ struct EmitParams {
   float c_ce, c_kl, inv_acc;
   uint16_t* dl;             // or null
   int64_t ldd;
+  // with drows, token t's dl goes to row drows[t] of ndl; a token whose drows is outside [0, ndl)
+  // has none, and its teacher row is not read
+  const int64_t* drows;
+  int64_t ndl;
   int64_t n, v;
   int vt;
   float* asum;              // [vt][2][rows]: each 128-entry half tile's sum min(p, t)
@@ -102,7 +106,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // Workgroup: step s (tokens 32 s .. + 31 of both 128-token halves) of one 256 x 256 tile.
 // Memory-bound: 4 + 2 bytes read and 2 written per entry (bf16 teacher), every load of a wave
 // issued before its first use (24 KB a wave, 12 waves a CU).
-template <typename TT, bool LSE>
+template <typename TT, bool LSE, bool MAP>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(TT) == 2 ? 3 : 2)))
 void emit_tiles_kernel(EmitParams p) {
   using R = Rows<TT>;
@@ -126,6 +130,14 @@ void emit_tiles_kernel(EmitParams p) {
     }
     return;
   }
+  // this lane's token's row of dl, -1: none (n and ndl are below 2^31); a wave without any leaves,
+  // its tokens' sums are not read
+  int dmine = (int)t;
+  if (MAP) {
+    const int64_t m = t < p.n ? p.drows[t] : -1;
+    dmine = m >= 0 && m < p.ndl ? (int)m : -1;
+    if (!__any(dmine >= 0)) return;
+  }
   lds_t* const lds = (lds_t*)lds_raw[wv];
   const bool full = vb + 128 <= p.v;
 
@@ -144,6 +156,9 @@ void emit_tiles_kernel(EmitParams p) {
   for (int i = 0; i < R::kLoads; ++i) {
     int64_t tr = tb + R::row(i, lane);
     tr = tr < p.n ? tr : p.n - 1;
+    // a row without dl reads the step's first (a branch here made every load wait: 8.5 ms at
+    // N = 2048 for 0.5)
+    if (MAP) tr = __shfl(dmine, R::row(i, lane)) >= 0 ? tr : tb;
     if (p.trows) {
       tr = p.trows[tr];
       tr = tr >= 0 && tr < p.nt ? tr : 0;   // its log-normaliser is NaN
@@ -219,8 +234,9 @@ void emit_tiles_kernel(EmitParams p) {
   for (int i = 0; i < 8; ++i) {
     const int row = 4 * i + (lane >> 4);
     const u32x4_t x = R::out(lds, row, c);
-    if (tb + row < p.n && ocol < p.v)
-      __builtin_nontemporal_store(x, reinterpret_cast<u32x4_t*>(p.dl + (tb + row) * p.ldd + ocol));
+    const int64_t dr = MAP ? (int64_t)__shfl(dmine, row) : tb + row;
+    if ((MAP ? dr >= 0 : dr < p.n) && ocol < p.v)
+      __builtin_nontemporal_store(x, reinterpret_cast<u32x4_t*>(p.dl + dr * p.ldd + ocol));
   }
 }
 
@@ -232,7 +248,8 @@ void emit_tiles_kernel(EmitParams p) {
 template <bool LSE, int kSumRows>
 __global__ __launch_bounds__(256) void emit_rows_kernel(const float* __restrict__ asum, const float* __restrict__ ksum,
                                                         int64_t rows, int vt, int splits, int64_t n,
-                                                        float* __restrict__ row_stats) {
+                                                        float* __restrict__ row_stats, int64_t* __restrict__ drows,
+                                                        int64_t ndl) {
   extern __shared__ float sh[];   // [LSE ? 2 : 1][splits][16]
   const int rl = threadIdx.x % kSumRows, l = threadIdx.x / kSumRows;
   const int64_t r = (int64_t)blockIdx.x * kSumRows + rl;
@@ -254,9 +271,16 @@ __global__ __launch_bounds__(256) void emit_rows_kernel(const float* __restrict_
   }
   __syncthreads();
   if (l > 0 || r >= n) return;
+  float* rs = row_stats + r * kRowStatWidth;
+  if (drows && (drows[r] < 0 || drows[r] >= ndl)) {
+    // a row without dl: accept 0, or NaN (and marked) where its dl is 0 * NaN
+    const float none = accept_rate_of(0.f, rs[kLseZ], rs[kLseU]);
+    rs[kAccept] = none;
+    drows[r] = none == 0.f ? -1 : kRowNan;
+    return;
+  }
   float a = sh[rl];
   for (int sp = 1; sp < splits; ++sp) a += sh[sp * kSumRows + rl];
-  float* rs = row_stats + r * kRowStatWidth;
   rs[kAccept] = accept_rate_of(a, rs[kLseZ], rs[kLseU]);
   if (LSE) {
     float k = sh[splits * kSumRows + rl];
@@ -265,12 +289,12 @@ __global__ __launch_bounds__(256) void emit_rows_kernel(const float* __restrict_
   }
 }
 
-template <typename TT, bool LSE>
+template <typename TT, bool LSE, bool MAP>
 hipError_t launch(const EmitParams& p, int splits, float* row_stats, hipStream_t st) {
   const int tt = (int)((p.n + 255) / 256);
   {
     NS_TIMED("head_emit", st);
-    hipLaunchKernelGGL((emit_tiles_kernel<TT, LSE>), dim3((unsigned)p.vt * 4, (unsigned)tt), dim3(kThreads), 0, st, p);
+    hipLaunchKernelGGL((emit_tiles_kernel<TT, LSE, MAP>), dim3((unsigned)p.vt * 4, (unsigned)tt), dim3(kThreads), 0, st, p);
     if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
   NS_TIMED("row_parts", st);
@@ -279,10 +303,10 @@ hipError_t launch(const EmitParams& p, int splits, float* row_stats, hipStream_t
   const size_t lds = (size_t)splits * rows * sizeof(float) * (LSE ? 2 : 1);
   if (rows == 4)
     hipLaunchKernelGGL((emit_rows_kernel<LSE, 4>), grid, dim3(256), lds, st, p.asum, p.ksum, p.rows, p.vt, splits, p.n,
-                       row_stats);
+                       row_stats, const_cast<int64_t*>(p.drows), p.ndl);
   else
     hipLaunchKernelGGL((emit_rows_kernel<LSE, 16>), grid, dim3(256), lds, st, p.asum, p.ksum, p.rows, p.vt, splits,
-                       p.n, row_stats);
+                       p.n, row_stats, const_cast<int64_t*>(p.drows), p.ndl);
   return hipGetLastError();
 }
 
@@ -295,7 +319,8 @@ size_t emit_workspace_bytes(int64_t n, int64_t v) {
 }
 
 hipError_t emit_from_tiles(void* ws, const void* teacher, int tdt, int64_t ldt, const TeacherSpec& ts, int64_t v,
-                           const SlotArgs& a, int splits, void* dl, int64_t ldd, float* row_stats, hipStream_t st) {
+                           const SlotArgs& a, int splits, void* dl, int64_t ldd, int64_t* drows, int64_t ndl,
+                           float* row_stats, hipStream_t st) {
   EmitParams p = {};
   const int64_t tt = (a.n + 255) / 256;
   p.vt = (int)((v + 255) / 256);
@@ -311,10 +336,16 @@ hipError_t emit_from_tiles(void* ws, const void* teacher, int tdt, int64_t ldt, 
   p.labels = a.labels; p.weights = a.weights; p.row_stats = row_stats;
   p.c_ce = a.c_ce; p.c_kl = a.c_kl; p.inv_acc = a.inv_acc;
   p.dl = static_cast<uint16_t*>(dl); p.ldd = ldd;
+  p.drows = drows; p.ndl = ndl;
   p.n = a.n; p.v = v;
+  if (drows)
+    return tdt == kBF16 ? launch<uint16_t, false, true>(p, splits, row_stats, st)
+                        : launch<float, false, true>(p, splits, row_stats, st);
   if (tdt == kBF16)
-    return ts.lse ? launch<uint16_t, true>(p, splits, row_stats, st) : launch<uint16_t, false>(p, splits, row_stats, st);
-  return ts.lse ? launch<float, true>(p, splits, row_stats, st) : launch<float, false>(p, splits, row_stats, st);
+    return ts.lse ? launch<uint16_t, true, false>(p, splits, row_stats, st)
+                  : launch<uint16_t, false, false>(p, splits, row_stats, st);
+  return ts.lse ? launch<float, true, false>(p, splits, row_stats, st)
+                : launch<float, false, false>(p, splits, row_stats, st);
 }
 
 }  // namespace ns

@@ -1587,9 +1587,12 @@ size_t lmhead_min_workspace_bytes(int64_t n, int64_t v) {
 
 size_t lmhead_workspace_bytes(int64_t n, int64_t v, int64_t d) {
   const size_t least = lmhead_min_workspace_bytes(n, v);
-  if (n == 0 || v == 0 || !keeps_tiles(n, v, d)) return least;
+  return n == 0 || v == 0 || !keeps_tiles(n, v, d) ? least : lmhead_rows_workspace_bytes(n, v);
+}
+
+size_t lmhead_rows_workspace_bytes(int64_t n, int64_t v) {
   const int64_t rows = window_rows(n, v);
-  return align_up(least, 256) + emit_workspace_bytes(n < rows ? n : rows, v);
+  return align_up(lmhead_min_workspace_bytes(n, v), 256) + emit_workspace_bytes(n < rows ? n : rows, v);
 }
 
 namespace {
@@ -1605,6 +1608,8 @@ struct HeadArgs {
   SlotArgs a;
   uint16_t* dl;
   int64_t ldd;
+  int64_t* drows;   // dl row of each row (null: its own) among ndl
+  int64_t ndl;
   float* row_stats;
 };
 
@@ -1622,7 +1627,8 @@ HeadArgs rows_of(const HeadArgs& x, MarkovFactors* f, int64_t r0, int64_t rows) 
     if (x.ts.lse) w.ts.lse += r0;
     w.ts.nt = rows;
   }
-  if (x.dl) w.dl += r0 * x.ldd;
+  if (x.drows) w.drows += r0;
+  else if (x.dl) w.dl += r0 * x.ldd;
   w.row_stats += r0 * kRowStatWidth;
   if (x.factors) {
     *f = *x.factors;
@@ -1688,7 +1694,8 @@ hipError_t head_window(const HeadArgs& x, int parts, bool keep, void* ws, size_t
   }
   if (!(parts & kHeadEmit)) return hipSuccess;
   if (keep)
-    return emit_from_tiles(zws, x.teacher, x.tdt, x.ldt, x.ts, x.v, x.a, pl.splits, x.dl, x.ldd, x.row_stats, st);
+    return emit_from_tiles(zws, x.teacher, x.tdt, x.ldt, x.ts, x.v, x.a, pl.splits, x.dl, x.ldd, x.drows, x.ndl,
+                           x.row_stats, st);
   if ((e = head_emit_window(p, pl, x.tdt, st)) != hipSuccess) return e;
   return launch_finalize(w.parta, pl.splits, x.a, x.row_stats, nullptr, st, p.tlse ? w.partk : nullptr);
 }
@@ -1716,13 +1723,17 @@ HeadArgs head_args(const void* hidden, int64_t ldh, const void* weight, int64_t 
 hipError_t lmhead_forward(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const void* markov,
                           int64_t ldm, const MarkovFactors* factors, const void* teacher, int tdt, int64_t ldt,
                           int64_t d, int64_t v, const SlotArgs& a, const TeacherSpec* ts, void* dl, int64_t ldd,
-                          float* row_stats, float* metrics, void* ws, size_t ws_bytes, hipStream_t st, int parts) {
+                          float* row_stats, float* metrics, void* ws, size_t ws_bytes, hipStream_t st, int parts,
+                          int64_t* drows, int64_t ndl) {
   if (a.n == 0) return metrics ? launch_finalize(nullptr, 1, a, row_stats, metrics, st) : hipSuccess;
-  const HeadArgs x = head_args(hidden, ldh, weight, ldw, markov, ldm, factors, teacher, tdt, ldt, d, v, a, ts, dl,
-                               ldd, row_stats);
+  HeadArgs x = head_args(hidden, ldh, weight, ldw, markov, ldm, factors, teacher, tdt, ldt, d, v, a, ts, dl, ldd,
+                         row_stats);
+  x.drows = drows;
+  x.ndl = ndl;
   const size_t least = lmhead_min_workspace_bytes(a.n, v);
   // pass 2 reads pass 1's values when both run here and the workspace holds them
-  const bool keep = parts == kHeadParts && keeps_tiles(a.n, v, d) && ws_bytes >= lmhead_workspace_bytes(a.n, v, d);
+  const bool keep = drows || (parts == kHeadParts && keeps_tiles(a.n, v, d) &&
+                              ws_bytes >= lmhead_workspace_bytes(a.n, v, d));
   const int64_t rows = rows_per_window(a.n, v, ws_bytes);
   for (int64_t r0 = 0; r0 < a.n; r0 += rows) {
     MarkovFactors f;

@@ -90,6 +90,7 @@ struct MarkovFactors {
 size_t lmhead_required_bytes(int64_t n, int64_t v);
 size_t lmhead_min_workspace_bytes(int64_t n, int64_t v);
 size_t lmhead_workspace_bytes(int64_t n, int64_t v, int64_t d);
+size_t lmhead_rows_workspace_bytes(int64_t n, int64_t v);   // with drows: always with the tile values
 // Raises the dynamic-LDS limit of every head instantiation lmhead_forward can launch, on the
 // current device (done lazily at launch otherwise; this lets a caller do it before capture).
 hipError_t lmhead_forward_prepare();
@@ -101,7 +102,11 @@ hipError_t lmhead_forward(const void* hidden, int64_t ldh, const void* weight, i
                           const void* markov, int64_t ldm, const MarkovFactors* factors, const void* teacher,
                           int tdt, int64_t ldt, int64_t d, int64_t v, const SlotArgs& a, const TeacherSpec* ts,
                           void* dl, int64_t ldd, float* row_stats, float* metrics, void* ws, size_t ws_bytes,
-                          hipStream_t st, int parts = kHeadParts);
+                          hipStream_t st, int parts = kHeadParts, int64_t* drows = nullptr, int64_t ndl = 0);
+// dl row index of every row that is supervised (valid or a non-zero weight), in order, -1 for
+// the others; count[0] = how many
+hipError_t kept_rows(const float* weights, const uint8_t* valid, int64_t n, int64_t* index, int64_t* count,
+                     hipStream_t st);
 
 // ---- second pass over kept tile values (emit.hip) ------------------------------
 // One 256 x 256 tile of draft logits (fp32, Markov addend included) as pass 1's accumulators hold
@@ -113,10 +118,15 @@ constexpr int64_t kZTile = 256 * 256;
 // partial sums after them.
 size_t emit_workspace_bytes(int64_t n, int64_t v);
 // accept rates (with ts.lse also KL) into row_stats and dl (if not NULL) of a window of a.n rows;
-// `splits`: the vocab splits whose order the row sums follow
+// `splits`: the vocab splits whose order the row sums follow.  With drows (ts.lse null) row t's dl
+// goes to row drows[t] of ndl; rows mapped outside [0, ndl) have none, their accept rate is 0 (NaN
+// when a log-normaliser is not finite) and their drows becomes -1 (kRowNan).
+constexpr int64_t kRowNan = INT64_MIN;
 hipError_t emit_from_tiles(void* ws, const void* teacher, int tdt, int64_t ldt, const TeacherSpec& ts, int64_t v,
-                           const SlotArgs& a, int splits, void* dl, int64_t ldd, float* row_stats, hipStream_t st);
-// dst row r = src row map[r] (row_bytes bytes), or zeros where map[r] is outside [0, n_src)
+                           const SlotArgs& a, int splits, void* dl, int64_t ldd, int64_t* drows, int64_t ndl,
+                           float* row_stats, hipStream_t st);
+// dst row r = src row map[r] (row_bytes bytes), or zeros where map[r] is outside [0, n_src), or
+// bytes of 0xFF (NaN in bf16 and fp32) where map[r] is kRowNan
 hipError_t copy_rows(const void* src, int64_t ld_src, int64_t n_src, const int64_t* map, int64_t n_dst,
                      int64_t row_bytes, void* dst, int64_t ld_dst, hipStream_t st);
 // Pass 2 of lmhead_forward alone: dl for a.inv_acc from the row_stats a forward over the

@@ -111,8 +111,8 @@ class _HeadInputs:
 
 @dataclass
 class _Compact:
-    """Pass 2 ran on a subset of the rows (``skip_masked_rows``): their dl rows, in order,
-    and for each of the N rows its index among them or -1."""
+    """dl was formed for a subset of the rows (``skip_masked_rows``): their dl rows, in order,
+    and for each of the N rows its index among them, or -1 (a zero row) or NS_ROW_NAN."""
 
     dl: torch.Tensor       # [m, V] bf16
     index: torch.Tensor    # [N] int64
@@ -162,14 +162,12 @@ def lm_head_ce_kl_loss(hidden, lm_head_weight, target_logits, prepared, objectiv
     into the GEMM as a second K segment, and the backward can form its gradients.
 
     ``skip_masked_rows=True`` (dense or no Markov addend, plain teacher logits): pass 1 runs on
-    every row, then pass 2 and the backward's dh GEMM only on the rows whose dl is not all
-    zero -- the supervised ones, and unsupervised ones whose log-normalisers are not finite
-    (their dl is the reference's 0 * NaN).  An unsupervised row with finite statistics has
-    dl = +0 and contributes (accept_rate * 0) to accept_len, exactly as in the reference, so the
-    outputs are those of the full pass (dl, CE/KL sums bit for bit; accept rates may differ in
-    their last bit, from a different split of the vocabulary).  Choosing the rows reads their
-    count on the host (one synchronisation), so this path cannot be captured into a graph; row
-    statistics of the skipped rows carry accept_rate 0.
+    every row, then pass 2 and the backward's dh GEMM only on the supervised rows.  An
+    unsupervised row with finite statistics has dl = +0 and contributes (accept_rate * 0) to
+    accept_len, exactly as in the reference (one whose log-normalisers are not finite has the
+    reference's 0 * NaN), so the outputs are those of the full pass, dl and the metrics bit for
+    bit.  Sizing dl reads the supervised rows' count on the host (one synchronisation), so this
+    path cannot be captured into a graph; row statistics of the skipped rows carry accept_rate 0.
     """
     o = objective
     if accumulation_steps < 1:
@@ -206,8 +204,10 @@ def lm_head_ce_kl_loss(hidden, lm_head_weight, target_logits, prepared, objectiv
         raise ValueError("pass either markov_logits or markov factors, not both")
     wts, y, valid, k = _slot_inputs(prepared, n, device)
     if skip_masked_rows and markov is None and targs is None and emit_dlogits:
-        return _forward_skipping_masked(o, lm_head_weight, hidden.shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts,
-                                        valid, k, accumulation_steps, device)
+        out = _forward_skipping_masked(o, lm_head_weight, hidden.shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts,
+                                       valid, k, accumulation_steps, device)
+        if out is not None:
+            return out
     metrics = torch.empty(6, dtype=torch.float32, device=device)
     row_stats = torch.empty((n, 8), dtype=torch.float32, device=device)
     dl = torch.empty((n, vocab), dtype=torch.bfloat16, device=device) if emit_dlogits else None
@@ -236,62 +236,37 @@ def lm_head_ce_kl_loss(hidden, lm_head_weight, target_logits, prepared, objectiv
 
 def _forward_skipping_masked(o, lm_head_weight, hidden_shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts, valid, k,
                              accumulation_steps, device):
-    """lm_head_ce_kl_loss(skip_masked_rows=True): pass 1 on every row, pass 2 on the rows whose
-    dl is not all zero -- their hidden and Markov rows gathered into compact copies
-    (ns_copy_rows), their teacher rows read in place through the teacher-row gather of the
-    kernels' loads -- the metrics from every row's statistics.  The compact dl is kept with
-    each row's index among the kept ones; the backward runs the dh GEMM on it and scatters dh
-    among zero rows, and forms the [N, V] dl (zero rows between) only for a caller that asks
-    for it (return_dlogits, final_norm).  At C3 (18,326 of 32,768 rows kept) reading the teacher rows in place instead of
-    copying them saved 3.9 of 12.7 ms of copies per step and left pass 2's time unchanged."""
+    """lm_head_ce_kl_loss(skip_masked_rows=True): pass 1 on every row, dl formed from its values for
+    the supervised rows only, into a compact [rows, V] dl (ns_lmhead_ce_kl_fwd_rows) that is kept
+    with each row's index in it; the backward runs the dh GEMM on it and scatters dh among zero
+    rows, and forms the [N, V] dl (zero rows between) only for a caller that asks for it
+    (return_dlogits, final_norm).  An unsupervised row whose statistics are not finite has a NaN dl
+    and dh row: its index says so.  Returns None when every row is supervised."""
     lib = _lib.load()
     st = _lib.stream(device)
     n = h.shape[0]
     vocab, d = lm_head_weight.shape
-    inv_acc = 1.0 / accumulation_steps
-
-    def part(which, hh, ldhh, mm, ldmm, uu, lduu, yy, ww, rows, dl, row_stats, targs=None):
-        ws = _lib.workspace(_lib.NS_WS_LMHEAD_MIN, rows, vocab, d, device)
-        status = lib.ns_lmhead_ce_kl_fwd_part(
-            which, _lib.ptr(hh), ldhh, _lib.ptr(w), ldw, _lib.ptr(mm), ldmm, _lib.ptr(uu), _lib.dtype_code(uu), lduu,
-            ctypes.byref(targs) if targs is not None else None, _lib.ptr(yy), _lib.ptr(ww), rows, d, vocab,
-            float(o.ce), float(o.kl), inv_acc, _lib.ptr(dl), vocab, _lib.ptr(row_stats), _lib.ptr(ws), ws.numel(), st)
-        _lib.check(status, "ns_lmhead_ce_kl_fwd_part")
-
-    row_stats = torch.empty((n, 8), dtype=torch.float32, device=device)
-    part(_lib.NS_PART_STATS, h, ldh, m, ldm, u, ldu, y, wts, n, None, row_stats)
-    # rows whose pass-2 outputs are not all zero: supervised ones, and unsupervised ones whose
-    # log-normalisers are not finite (the reference's dl there is 0 * NaN, its accept 0 * NaN)
-    need = (valid != 0) | (wts != 0) | ~torch.isfinite(row_stats[:, 0]) | ~torch.isfinite(row_stats[:, 1])
-    act = torch.nonzero(need).reshape(-1)   # reads the count on the host: it sizes the compacted pass
-    rows = act.numel()
-    dl = compact = None
+    index = torch.empty(n + 1, dtype=torch.int64, device=device)
+    _lib.check(lib.ns_kept_rows(_lib.ptr(wts), _lib.ptr(valid), n, _lib.ptr(index), _lib.ptr(index[n:]), st),
+               "ns_kept_rows")
+    rows = int(index[n])   # read on the host: it sizes dl
     if rows == n:
-        dl = torch.empty((n, vocab), dtype=torch.bfloat16, device=device)
-        part(_lib.NS_PART_EMIT, h, ldh, m, ldm, u, ldu, y, wts, n, dl, row_stats)
-    else:
-        hc = _lib.copy_rows(h, act, rows, torch.empty((rows, d), dtype=h.dtype, device=device))
-        mc = _lib.copy_rows(m, act, rows, torch.empty((rows, vocab), dtype=m.dtype, device=device)) \
-            if m is not None else None
-        # the teacher rows are read in place, gathered in the kernels' loads
-        targs = _lib.TeacherArgs(_lib.ptr(act), u.shape[0], None)
-        rs = row_stats.index_select(0, act)
-        dlc = torch.empty((rows, vocab), dtype=torch.bfloat16, device=device)
-        part(_lib.NS_PART_EMIT, hc, d, mc, vocab, u, ldu, y.index_select(0, act), wts.index_select(0, act), rows,
-             dlc, rs, targs)
-        del hc, mc
-        row_stats.index_copy_(0, act, rs)
-        row_stats[:, 4].masked_fill_(~need, 0.0)   # (accept_rate * valid) is 0 there either way
-        index = torch.full((n,), -1, dtype=torch.int64, device=device)
-        index.index_copy_(0, act, torch.arange(rows, dtype=torch.int64, device=device))
-        compact = _Compact(dlc, index)   # the [N, V] dl is formed only if a caller asks for it
+        return None
+    index = index[:n]
     metrics = torch.empty(6, dtype=torch.float32, device=device)
-    status = lib.ns_objective_metrics(_lib.ptr(row_stats), _lib.ptr(wts), _lib.ptr(valid), n, k, float(o.ce),
-                                      float(o.kl), _lib.ptr(metrics), st)
-    _lib.check(status, "ns_objective_metrics")
+    row_stats = torch.empty((n, 8), dtype=torch.float32, device=device)
+    dl = torch.empty((rows, vocab), dtype=torch.bfloat16, device=device)
+    ws = _lib.workspace(_lib.NS_WS_LMHEAD_ROWS, n, vocab, d, device)
+    status = lib.ns_lmhead_ce_kl_fwd_rows(
+        _lib.ptr(h), ldh, _lib.ptr(w), ldw, _lib.ptr(m), ldm, _lib.ptr(u), _lib.dtype_code(u), ldu, None, _lib.ptr(y),
+        _lib.ptr(wts), _lib.ptr(valid), n, d, vocab, k, float(o.ce), float(o.kl), 1.0 / accumulation_steps,
+        _lib.ptr(dl), vocab, _lib.ptr(index), rows, _lib.ptr(row_stats), _lib.ptr(metrics), _lib.ptr(ws), ws.numel(),
+        st)
+    _lib.check(status, "ns_lmhead_ce_kl_fwd_rows")
     inputs = _HeadInputs(h, ldh, w, ldw, m, ldm, None, u, ldu, None, None, y, wts)
     shape = tuple(hidden_shape[:-1]) + (vocab,)
-    saved = HeadActivations(o, lm_head_weight, row_stats, dl, accumulation_steps, shape, None, inputs, compact)
+    saved = HeadActivations(o, lm_head_weight, row_stats, None, accumulation_steps, shape, None, inputs,
+                            _Compact(dl, index))
     return LossMetrics.from_buffer(metrics), saved
 
 
