@@ -1,5 +1,5 @@
 // Row copies by an index map: dst row r = src row map[r], zeros where map[r] is outside
-// [0, n_src) (NaN where it is kRowNan).  The fused head keeps dl and runs the dh GEMM on the rows
+// [0, n_src) (NaN where it is kRowNan).  The fused head forms dl and runs the dh GEMM on the rows
 // whose outputs are not all zero (head.lm_head_ce_kl_loss(skip_masked_rows=True)): the compact dh
 // (and, on request, dl) is scattered back with zero rows between.  HBM-bound: each byte is read
 // and written once, with non-temporal 16-byte accesses (the rows are not read again soon).

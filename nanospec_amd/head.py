@@ -165,8 +165,9 @@ def lm_head_ce_kl_loss(hidden, lm_head_weight, target_logits, prepared, objectiv
     every row, then pass 2 and the backward's dh GEMM only on the supervised rows.  An
     unsupervised row with finite statistics has dl = +0 and contributes (accept_rate * 0) to
     accept_len, exactly as in the reference (one whose log-normalisers are not finite has the
-    reference's 0 * NaN), so the outputs are those of the full pass, dl and the metrics bit for
-    bit.  Sizing dl reads the supervised rows' count on the host (one synchronisation), so this
+    reference's 0 * NaN), so the outputs are those of the full pass, dl and the CE/KL sums bit for
+    bit (accept rates may differ in their last bit where the kept rows go through a pass of their
+    own).  Sizing dl reads the supervised rows' count on the host (one synchronisation), so this
     path cannot be captured into a graph; row statistics of the skipped rows carry accept_rate 0.
     """
     o = objective
@@ -204,8 +205,9 @@ def lm_head_ce_kl_loss(hidden, lm_head_weight, target_logits, prepared, objectiv
         raise ValueError("pass either markov_logits or markov factors, not both")
     wts, y, valid, k = _slot_inputs(prepared, n, device)
     if skip_masked_rows and markov is None and targs is None and emit_dlogits:
-        out = _forward_skipping_masked(o, lm_head_weight, hidden.shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts,
-                                       valid, k, accumulation_steps, device)
+        skipping = _forward_skipping_masked if _skips_on_values(n, vocab, d) else _forward_compact_rows
+        out = skipping(o, lm_head_weight, hidden.shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts, valid, k,
+                       accumulation_steps, device)
         if out is not None:
             return out
     metrics = torch.empty(6, dtype=torch.float32, device=device)
@@ -232,6 +234,15 @@ def lm_head_ce_kl_loss(hidden, lm_head_weight, target_logits, prepared, objectiv
     shape = tuple(hidden.shape[:-1]) + (vocab,)
     saved = HeadActivations(o, lm_head_weight, row_stats, dl, accumulation_steps, shape, markov, inputs)
     return LossMetrics.from_buffer(metrics), saved
+
+
+def _skips_on_values(n: int, vocab: int, d: int) -> bool:
+    """Whether ``skip_masked_rows`` forms dl from pass 1's values (8 bytes moved per entry of every
+    row) or runs the GEMM again on the kept rows.  Steps with half of the rows supervised, values /
+    GEMM again, V = 248,320: N = 3500: d = 256 3.28 / 3.06 ms, 512 3.84 / 3.55, 768 4.48 / 4.40,
+    1024 4.88 / 5.04, 2048 6.80 / 7.58; N = 1001: 256 0.99 / 1.25, 1024 1.59 / 1.82; N = 3500,
+    V = 65,536: 256 0.97 / 1.06, 512 1.09 / 1.19."""
+    return d >= 896 or n * vocab <= 1 << 28
 
 
 def _forward_skipping_masked(o, lm_head_weight, hidden_shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts, valid, k,
@@ -267,6 +278,62 @@ def _forward_skipping_masked(o, lm_head_weight, hidden_shape, h, ldh, w, ldw, m,
     shape = tuple(hidden_shape[:-1]) + (vocab,)
     saved = HeadActivations(o, lm_head_weight, row_stats, None, accumulation_steps, shape, None, inputs,
                             _Compact(dl, index))
+    return LossMetrics.from_buffer(metrics), saved
+
+
+def _forward_compact_rows(o, lm_head_weight, hidden_shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts, valid, k,
+                          accumulation_steps, device):
+    """skip_masked_rows where a second GEMM over the kept rows costs less than pass 1's values
+    written and read (``_skips_on_values``): pass 1 on every row, then pass 2 on the rows whose dl
+    is not all zero (supervised, or with statistics that are not finite), their hidden and Markov
+    rows gathered into compact copies (ns_copy_rows), their teacher rows read in place."""
+    lib = _lib.load()
+    st = _lib.stream(device)
+    n = h.shape[0]
+    vocab, d = lm_head_weight.shape
+    inv_acc = 1.0 / accumulation_steps
+
+    def part(which, hh, ldhh, mm, ldmm, uu, lduu, yy, ww, rows, dl, row_stats, targs=None):
+        ws = _lib.workspace(_lib.NS_WS_LMHEAD_MIN, rows, vocab, d, device)
+        status = lib.ns_lmhead_ce_kl_fwd_part(
+            which, _lib.ptr(hh), ldhh, _lib.ptr(w), ldw, _lib.ptr(mm), ldmm, _lib.ptr(uu), _lib.dtype_code(uu), lduu,
+            ctypes.byref(targs) if targs is not None else None, _lib.ptr(yy), _lib.ptr(ww), rows, d, vocab,
+            float(o.ce), float(o.kl), inv_acc, _lib.ptr(dl), vocab, _lib.ptr(row_stats), _lib.ptr(ws), ws.numel(), st)
+        _lib.check(status, "ns_lmhead_ce_kl_fwd_part")
+
+    row_stats = torch.empty((n, 8), dtype=torch.float32, device=device)
+    part(_lib.NS_PART_STATS, h, ldh, m, ldm, u, ldu, y, wts, n, None, row_stats)
+    # (the reference's dl of an unsupervised row is 0 * NaN there, its accept 0 * NaN)
+    need = (valid != 0) | (wts != 0) | ~torch.isfinite(row_stats[:, 0]) | ~torch.isfinite(row_stats[:, 1])
+    act = torch.nonzero(need).reshape(-1)   # reads the count on the host: it sizes the compacted pass
+    rows = act.numel()
+    dl = compact = None
+    if rows == n:
+        dl = torch.empty((n, vocab), dtype=torch.bfloat16, device=device)
+        part(_lib.NS_PART_EMIT, h, ldh, m, ldm, u, ldu, y, wts, n, dl, row_stats)
+    else:
+        hc = _lib.copy_rows(h, act, rows, torch.empty((rows, d), dtype=h.dtype, device=device))
+        mc = _lib.copy_rows(m, act, rows, torch.empty((rows, vocab), dtype=m.dtype, device=device)) \
+            if m is not None else None
+        # the teacher rows are read in place, gathered in the kernels' loads
+        targs = _lib.TeacherArgs(_lib.ptr(act), u.shape[0], None)
+        rs = row_stats.index_select(0, act)
+        dlc = torch.empty((rows, vocab), dtype=torch.bfloat16, device=device)
+        part(_lib.NS_PART_EMIT, hc, d, mc, vocab, u, ldu, y.index_select(0, act), wts.index_select(0, act), rows,
+             dlc, rs, targs)
+        del hc, mc
+        row_stats.index_copy_(0, act, rs)
+        row_stats[:, 4].masked_fill_(~need, 0.0)   # (accept_rate * valid) is 0 there either way
+        index = torch.full((n,), -1, dtype=torch.int64, device=device)
+        index.index_copy_(0, act, torch.arange(rows, dtype=torch.int64, device=device))
+        compact = _Compact(dlc, index)   # the [N, V] dl is formed only if a caller asks for it
+    metrics = torch.empty(6, dtype=torch.float32, device=device)
+    status = lib.ns_objective_metrics(_lib.ptr(row_stats), _lib.ptr(wts), _lib.ptr(valid), n, k, float(o.ce),
+                                      float(o.kl), _lib.ptr(metrics), st)
+    _lib.check(status, "ns_objective_metrics")
+    inputs = _HeadInputs(h, ldh, w, ldw, m, ldm, None, u, ldu, None, None, y, wts)
+    shape = tuple(hidden_shape[:-1]) + (vocab,)
+    saved = HeadActivations(o, lm_head_weight, row_stats, dl, accumulation_steps, shape, None, inputs, compact)
     return LossMetrics.from_buffer(metrics), saved
 
 

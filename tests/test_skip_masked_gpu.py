@@ -177,3 +177,26 @@ def test_skip_with_final_norm_and_dl_formed_on_request(gpu_lib):
         (dxf, dlf, wgf), (dxs, dls, wgs) = out
         assert torch.equal(dlf, dls)
         assert torch.equal(dxf, dxs) and torch.equal(wgf, wgs)
+
+
+@pytest.mark.parametrize("on_values", [True, False])
+@pytest.mark.parametrize("fp32_teacher", [False, True])
+def test_both_ways_of_skipping_give_the_full_pass(gpu_lib, monkeypatch, on_values, fp32_teacher):
+    """dl from pass 1's values or from a second GEMM over the kept rows (the choice is by size), a
+    non-finite unsupervised row among them."""
+    monkeypatch.setattr(head, "_skips_on_values", lambda n, v, d: on_values)
+    n, d, v = 520, 320, 2184
+    hidden, weight, markov, teacher, slots = synthetic.head_inputs(n, d, v, 5701, DEV, ragged=True)
+    if fp32_teacher:
+        teacher = teacher.float()
+    o = Objective(block_size=8)
+    full, skip = _both(hidden, weight, markov, teacher, slots, o)
+    masked = _masked(slots)
+    _assert_same(full, skip, masked)
+    hidden = hidden.clone()
+    r = int(torch.nonzero(masked)[3])
+    hidden[r, 0] = float("inf")
+    (mf, _, dhf, dlf), (ms, _, dhs, dls) = _both(hidden, weight, markov, teacher, slots, o)
+    assert torch.isnan(dls[r]).all() and torch.isnan(dhs[r]).all()
+    assert torch.equal(torch.isnan(dlf), torch.isnan(dls)) and torch.equal(torch.isnan(dhf), torch.isnan(dhs))
+    assert torch.isnan(mf.accept_len_sum) and torch.isnan(ms.accept_len_sum)
