@@ -42,15 +42,21 @@ __device__ __forceinline__ void dma16(const char* base, uint32_t voff, lds_t* ds
 // no waits for one before LDS reads (with the builtin it waited for every outstanding fill
 // before a read it could not prove disjoint); the caller's own vmcnt waits must order each
 // fill before the reads of its data.  Same instruction, descriptor and LDS layout as dma16.
-// M0 is reserved to the compiler, which does not honour the clobber: a kernel using this
-// must not also use dma16 or anything else that sets M0 (the dh GEMM uses only this form).
+// M0 is reserved to the compiler, which does not honour a clobber: the block puts M0 back, so that
+// dma16 may be used in the same kernel.  One wait state lies between the M0 write and the load
+// that reads it (gfx9's LDS DMA; the compiler puts the same s_nop before dma16's).
 __device__ __forceinline__ void dma16_asm(const char* base, uint32_t voff, lds_t* dst) {
   typedef uint32_t u32x4s_t __attribute__((ext_vector_type(4)));
   const uint64_t b = reinterpret_cast<uint64_t>(base);
   const u32x4s_t rs = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, 0xffffffffu, 0x00020000u};
   const uint32_t m0v = (uint32_t)reinterpret_cast<uintptr_t>(dst);
-  asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(m0v)
-               : "memory", "m0");
+  uint32_t keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(voff), "s"(rs), "s"(m0v)
+      : "memory");
 }
 
 // A ROWS-row operand tile (128-byte rows) fetched straight into LDS (dma16).  Each of the
