@@ -72,9 +72,9 @@ def cpu_model() -> str:
 # library kernel symbol (demangled, as rocprofv3 prints it) -> the launch-site name the
 # library's own timer (ns_profile_*) uses
 KERNEL_NAMES = [
-    (r"head_kernel<0,", "head_stats"),
+    (r"head_kernel<0,|thin_kernel<0,", "head_stats"),
     (r"head_kernel<1,", "head_emit"),
-    (r"head_kernel<2,", "head_linear"),
+    (r"head_kernel<2,|thin_kernel<1,", "head_linear"),
     (r"sum_partials_kernel<[^,]+, (?:unsigned short|uint16_t)", "dh_reduce"),
     (r"dh_kernel", "dh_gemm"),
     (r"stream_stats_kernel", "stream_stats"),

@@ -448,14 +448,14 @@ int ns_lmhead_teacher_logits(const void* x, int64_t ldx, const int64_t* rows, in
   if (!aligned(x) || !aligned(weight) || !aligned(out) || ldx % 8 || ldw % 8 || ldo % 8)
     return fail(NS_EALIGN, "teacher head needs 16-byte aligned base pointers and rows");
   if (lse) {
-    const size_t need = ns::lmhead_linear_lse_workspace_bytes(n, v);
+    const size_t need = ns::linear_lse_required_bytes(n, v);
     if (n > 0 && (!workspace || workspace_bytes < need))
       return fail(NS_EWORKSPACE, "workspace of %zu bytes required (got %zu)", need, workspace_bytes);
     if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
       return fail(NS_EALIGN, "workspace must be 256-byte aligned");
   }
   return hip_status(ns::lmhead_linear_lse(x, ldx, rows, nx, weight, ldw, nullptr, 0, out, ldo, lse, n, v, d, workspace,
-                                          reinterpret_cast<hipStream_t>(stream)),
+                                          workspace_bytes, reinterpret_cast<hipStream_t>(stream)),
                     "ns_lmhead_teacher_logits");
 }
 

@@ -8,9 +8,8 @@
 // vocab entries of one wave as 16 KB, lane after lane.  A wave here takes one such block, so
 // each of its lanes holds the entries head_kernel<EMIT>'s lane holds and adds them in the same
 // order: dl and the accept sums are the same bits on either path.
-#include "ns_gemm.h"
-#include "ns_internal.h"
 #include "ns_profile.h"
+#include "ns_tiles.h"
 
 namespace ns {
 namespace {
@@ -39,69 +38,6 @@ struct EmitParams {
   float* ksum;              // likewise sum t (u - z) (LSE), or null
   int64_t rows;
 };
-
-// LDS image of a wave's 32 teacher rows (128 entries each), read back chunk by chunk (8
-// entries) and overwritten with dl.  bf16: 256-byte rows, chunk c at c ^ (row & 15), the
-// 8-byte halves of rows 16-31 swapped, so the 32 lanes of a read cover every bank once.
-// fp32: 512-byte rows of 16-byte quads, quad q at q ^ (row & 31).
-template <typename TT>
-struct Rows;
-template <>
-struct Rows<uint16_t> {
-  static constexpr int kBytes = 32 * 256;
-  static constexpr int kLoads = 8;        // 16-byte pieces per lane
-  static constexpr int kPer = 8;          // entries per piece
-  static __device__ __forceinline__ int row(int i, int lane) { return 4 * i + (lane >> 4); }
-  static __device__ __forceinline__ int piece(int lane) { return lane & 15; }
-  static __device__ __forceinline__ void put(lds_t* b, int i, int lane, u32x4_t x) {
-    const int r = row(i, lane), c = piece(lane);
-    if (i >= 4) x = u32x4_t{x[2], x[3], x[0], x[1]};
-    *reinterpret_cast<__attribute__((address_space(3))) u32x4_t*>(b + r * 256 + ((c ^ (r & 15)) << 4)) = x;
-  }
-  // byte offset of entries 8 k + 4 h .. + 3 of row r
-  static __device__ __forceinline__ int off(int k, int r, int h) {
-    return r * 256 + ((k ^ (r & 15)) << 4) + 8 * (h ^ (r >> 4));
-  }
-  static __device__ __forceinline__ void get(const lds_t* b, int k, int r, int h, float* u) {
-    const u32x2_t x = *reinterpret_cast<const __attribute__((address_space(3))) u32x2_t*>(b + off(k, r, h));
-    u[0] = bf16_lo(x[0]); u[1] = bf16_hi(x[0]);
-    u[2] = bf16_lo(x[1]); u[3] = bf16_hi(x[1]);
-  }
-  // dl chunk c of row r
-  static __device__ __forceinline__ u32x4_t out(const lds_t* b, int r, int c) {
-    const u32x4_t x = *reinterpret_cast<const __attribute__((address_space(3))) u32x4_t*>(b + r * 256 + ((c ^ (r & 15)) << 4));
-    return r >= 16 ? u32x4_t{x[2], x[3], x[0], x[1]} : x;
-  }
-};
-template <>
-struct Rows<float> {
-  static constexpr int kBytes = 32 * 512;
-  static constexpr int kLoads = 16;
-  static constexpr int kPer = 4;
-  static __device__ __forceinline__ int row(int i, int lane) { return 2 * i + (lane >> 5); }
-  static __device__ __forceinline__ int piece(int lane) { return lane & 31; }
-  static __device__ __forceinline__ void put(lds_t* b, int i, int lane, u32x4_t x) {
-    const int r = row(i, lane), q = piece(lane);
-    *reinterpret_cast<__attribute__((address_space(3))) u32x4_t*>(b + r * 512 + ((q ^ r) << 4)) = x;
-  }
-  static __device__ __forceinline__ int off(int k, int r, int h) { return r * 512 + (((2 * k + h) ^ r) << 4); }
-  static __device__ __forceinline__ void get(const lds_t* b, int k, int r, int h, float* u) {
-    const u32x4_t x = *reinterpret_cast<const __attribute__((address_space(3))) u32x4_t*>(b + off(k, r, h));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) u[e] = __uint_as_float(x[e]);
-  }
-  static __device__ __forceinline__ u32x4_t out(const lds_t* b, int r, int c) {
-    const u32x2_t lo = *reinterpret_cast<const __attribute__((address_space(3))) u32x2_t*>(b + off(c, r, 0));
-    const u32x2_t hi = *reinterpret_cast<const __attribute__((address_space(3))) u32x2_t*>(b + off(c, r, 1));
-    return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
-  }
-};
-
-// LDS written by some lanes of a wave, read by others of the same wave
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
 
 // Workgroup: step s (tokens 32 s .. + 31 of both 128-token halves) of one 256 x 256 tile.
 // Memory-bound: 4 + 2 bytes read and 2 written per entry (bf16 teacher), every load of a wave

@@ -29,6 +29,7 @@
 #include "ns_gemm.h"
 #include "ns_internal.h"
 #include "ns_profile.h"
+#include "ns_tiles.h"
 
 namespace ns {
 namespace {
@@ -482,37 +483,6 @@ constexpr int kTbadOff = kTrowOff + 256 * 4;        // [256] uint8: teacher (STO
 constexpr int kHrowOff = kTbadOff + 256;            // [256] int32 gathered B rows (MODE_STORE)
 constexpr int kHeadLdsBytes = kHrowOff + 256 * 4;
 static_assert(kHeadLdsBytes <= 160 * 1024, "head kernel LDS");
-
-__device__ __forceinline__ PairState half_merge(const PairState& s) {
-  PairState a, b;
-  half_pair(s.mz, a.mz, b.mz);
-  half_pair(s.sz, a.sz, b.sz);
-  half_pair(s.mu, a.mu, b.mu);
-  half_pair(s.su, a.su, b.su);
-  half_pair(s.A, a.A, b.A);
-  return pair_merge(a, b);
-}
-
-__device__ __forceinline__ LseState half_merge(const LseState& s) {
-  LseState a, b;
-  half_pair(s.m, a.m, b.m);
-  half_pair(s.s, a.s, b.s);
-  return lse_merge(a, b);
-}
-
-// One distribution's online (max, sum-exp) over W values.
-template <int W>
-__device__ __forceinline__ void lse_update(LseState& st, const float* z) {
-  float b = z[0];
-#pragma unroll
-  for (int i = 1; i < W; ++i) b = fmaxf(b, z[i]);
-  const float m = fmaxf(st.m, b);
-  const float ml = m * kLog2e;
-  float s = st.s * fast_exp2((st.m - m) * kLog2e);
-#pragma unroll
-  for (int i = 0; i < W; ++i) s += fast_exp2(__builtin_fmaf(z[i], kLog2e, -ml));
-  st = {m, s};
-}
 
 // pair_update<32> / lse_update<32> with f(g) called after each group of 8 exponentials
 // (the same arithmetic in the same order; the group's sums are pinned before the call)
@@ -1388,6 +1358,14 @@ int64_t window_rows(int64_t n, int64_t v) {
 // 2972 / 3030, 512 3296 / 3452; N = 448: 128 360 / 359, 256 382 / 417; N = 2048, V = 32,000:
 // 128 198 / 183, 256 210 / 211; N = 56: 128 147 / 200; N = 64, V = 8192, d = 64: 40 / 55.  The
 // fewer the values, the more of them the Infinity Cache (256 MB) still holds for pass 2.
+// Whether few rows' pass 1 and projection take thin.hip's kernel.  Projections here / with 256-token
+// tiles in microseconds, V = 248,320 unless said: d = 5120: n = 8 430 / 638, 64 470 / 635, 128
+// 527 / 649; d = 512: n = 8 45 / 86, 128 79 / 97; V = 8192, d = 5120: n = 8 49 / 92, 64 73 / 92;
+// V = 2048, d = 256, n = 8: 10 / 19.  With 65 to 128 rows two waves are the most a workgroup of 256
+// vocab rows holds, and smaller vocabularies lose: V = 100,000 287 / 294, 32,000 134 / 128, 8192
+// 118 / 92.
+bool thin_rows(int64_t n, int64_t v) { return n <= 64 || (n <= kThinRows && (v + BM - 1) / BM > kThinWide); }
+
 bool keeps_tiles(int64_t n, int64_t v, int64_t d) {
   const int64_t entries = n * v;
   return d >= (entries <= (int64_t(1) << 25) ? 64 : entries <= (int64_t(1) << 27) ? 192 : 320);
@@ -1592,7 +1570,8 @@ size_t lmhead_workspace_bytes(int64_t n, int64_t v, int64_t d) {
 
 size_t lmhead_rows_workspace_bytes(int64_t n, int64_t v) {
   const int64_t rows = window_rows(n, v);
-  return align_up(lmhead_min_workspace_bytes(n, v), 256) + emit_workspace_bytes(n < rows ? n : rows, v);
+  return align_up(lmhead_min_workspace_bytes(n, v), 256) + emit_workspace_bytes(n < rows ? n : rows, v) +
+         (thin_rows(n, v) ? thin_workspace_bytes(n, v) : 0);
 }
 
 namespace {
@@ -1674,8 +1653,8 @@ hipError_t head_emit_window(const HeadParams& p, const HeadPlan& pl, int tdt, hi
   return launch_head<MODE_EMIT, float, 0>(p, pl.grid, st, "head_emit");
 }
 
-// The passes of one window.
-hipError_t head_window(const HeadArgs& x, int parts, bool keep, void* ws, size_t least, hipStream_t st) {
+// The passes of one window; thin: all rows are few (thin_rows) and the workspace has room for it.
+hipError_t head_window(const HeadArgs& x, int parts, bool keep, bool thin, void* ws, size_t least, hipStream_t st) {
   const HeadPlan pl = head_plan(x.a.n, x.v);
   HeadWs w;
   window_ws_layout(x.a.n, pl.splits, ws, &w);
@@ -1683,7 +1662,15 @@ hipError_t head_window(const HeadArgs& x, int parts, bool keep, void* ws, size_t
   void* zws = static_cast<char*>(ws) + align_up(least, 256);
   p.z = keep ? static_cast<float*>(zws) : nullptr;
   hipError_t e = hipSuccess;
-  if (parts & kHeadStats) {
+  if ((parts & kHeadStats) && keep && thin) {
+    // the half tiles' partials lie after the kept values and pass 2's sums
+    RowPart* tpart = reinterpret_cast<RowPart*>(static_cast<char*>(zws) + emit_workspace_bytes(x.a.n, x.v));
+    const ThinHead th{x.hidden, x.weight, x.markov, x.ldh, x.ldw, x.ldm, x.d, x.v, x.factors};
+    e = thin_stats(th, x.a, x.ts, x.teacher, x.tdt, x.ldt, p.z, p.zy, tpart, st);
+    if (e != hipSuccess) return e;
+    e = launch_merge(tpart, p.zy, p.v, pl.splits, x.a, x.row_stats, st, p.tlse ? &x.ts : nullptr, pl.vt);
+    if (e != hipSuccess) return e;
+  } else if (parts & kHeadStats) {
     if (p.tlse)
       e = x.tdt == kBF16 ? head_stats_window<uint16_t, kTeacherLse>(p, pl, keep, x.a, &x.ts, x.row_stats, st)
                          : head_stats_window<float, kTeacherLse>(p, pl, keep, x.a, &x.ts, x.row_stats, st);
@@ -1738,7 +1725,7 @@ hipError_t lmhead_forward(const void* hidden, int64_t ldh, const void* weight, i
   for (int64_t r0 = 0; r0 < a.n; r0 += rows) {
     MarkovFactors f;
     const HeadArgs w = rows_of(x, &f, r0, a.n - r0 < rows ? a.n - r0 : rows);
-    if (const hipError_t e = head_window(w, parts, keep, ws, least, st); e != hipSuccess) return e;
+    if (const hipError_t e = head_window(w, parts, keep, thin_rows(a.n, v), ws, least, st); e != hipSuccess) return e;
   }
   // the rows' sums are in row_stats
   return metrics ? launch_finalize(nullptr, 1, a, row_stats, metrics, st) : hipSuccess;
@@ -1834,19 +1821,30 @@ hipError_t lmhead_backward_ext(const void* dl, int64_t ldd, const void* weight, 
 
 hipError_t lmhead_linear(const void* x, int64_t ldx, const void* weight, int64_t ldw, const void* addend,
                          int64_t lda, void* out, int64_t ldo, int64_t n, int64_t v, int64_t d, hipStream_t st) {
-  return lmhead_linear_lse(x, ldx, nullptr, 0, weight, ldw, addend, lda, out, ldo, nullptr, n, v, d, nullptr, st);
+  return lmhead_linear_lse(x, ldx, nullptr, 0, weight, ldw, addend, lda, out, ldo, nullptr, n, v, d, nullptr, 0, st);
 }
 
-size_t lmhead_linear_lse_workspace_bytes(int64_t n, int64_t v) {
+size_t linear_lse_required_bytes(int64_t n, int64_t v) {
   const HeadPlan pl = head_plan(n, v);
   return align_up((size_t)n * pl.splits * sizeof(RowPart), 256);
 }
 
+size_t lmhead_linear_lse_workspace_bytes(int64_t n, int64_t v) {
+  return linear_lse_required_bytes(n, v) + (thin_rows(n, v) ? thin_workspace_bytes(n, v) : 0);
+}
+
 hipError_t lmhead_linear_lse(const void* x, int64_t ldx, const int64_t* rows, int64_t nrows, const void* weight,
                              int64_t ldw, const void* addend, int64_t lda, void* out, int64_t ldo, float* lse,
-                             int64_t n, int64_t v, int64_t d, void* ws, hipStream_t st) {
+                             int64_t n, int64_t v, int64_t d, void* ws, size_t ws_bytes, hipStream_t st) {
   if (n == 0 || v == 0) return hipSuccess;
   const HeadPlan pl = head_plan(n, v);
+  if (thin_rows(n, v) && (!lse || ws_bytes >= lmhead_linear_lse_workspace_bytes(n, v))) {
+    const ThinHead th{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(weight),
+                      static_cast<const uint16_t*>(addend), ldx, ldw, lda, d, v, nullptr};
+    RowPart* tpart = lse ? reinterpret_cast<RowPart*>(static_cast<char*>(ws) + linear_lse_required_bytes(n, v)) : nullptr;
+    const hipError_t e = thin_store(th, rows, nrows, n, out, ldo, tpart, st);
+    return e != hipSuccess || !lse ? e : launch_lse_merge(tpart, pl.splits, n, lse, st, pl.vt);
+  }
   HeadParams p = {};
   p.hidden = static_cast<const uint16_t*>(x);
   p.weight = static_cast<const uint16_t*>(weight);

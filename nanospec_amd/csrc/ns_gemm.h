@@ -103,6 +103,9 @@ struct DmaTile {
   __device__ __forceinline__ void issue(const char* base, lds_t* dst, int wv, int i) const {
     dma16(base, off[i], dst + (wv * NI + i) * 1024);
   }
+  __device__ __forceinline__ void issue_asm(const char* base, lds_t* dst, int wv, int i) const {
+    dma16_asm(base, off[i], dst + (wv * NI + i) * 1024);
+  }
 };
 
 // B operand [K rows, cols] (cols contiguous) fetched straight into a row-major LDS stage

@@ -42,16 +42,18 @@ struct TeacherSpec {
   const float* lse;
 };
 // Merge first-pass partials part1[N][S] (+ z_y[N]) into row_stats (lse_z, lse_u, ce, kl, z_y).
-// With ts (its lse given) lse_u comes from ts and KL is left to the finalize.
+// With ts (its lse given) lse_u comes from ts and KL is left to the finalize.  tiles > 0: part1
+// holds the partials of half vocab tiles instead, [tiles][2][N], of which each of S splits takes a
+// contiguous range.
 hipError_t launch_merge(const RowPart* part1, const float* zy, int64_t v, int splits, const SlotArgs& a,
-                        float* row_stats, hipStream_t st, const TeacherSpec* ts = nullptr);
+                        float* row_stats, hipStream_t st, const TeacherSpec* ts = nullptr, int tiles = 0);
 // Sum accept partials parta[N][S], form block lengths and the six metrics; with partk
 // (pass-2 sums of t (u - z)), KL = sum partk - lse_u + lse_z first.  parta NULL: the metrics
 // alone, from complete row_stats; metrics NULL: the row sums alone.
 hipError_t launch_finalize(const float* parta, int splits, const SlotArgs& a, float* row_stats,
                            float* metrics, hipStream_t st, const float* partk = nullptr);
 // lse[t] = log-sum-exp from (max, sum-exp) partials part1[N][S] (mz, sz), fixed order.
-hipError_t launch_lse_merge(const RowPart* part1, int splits, int64_t n, float* lse, hipStream_t st);
+hipError_t launch_lse_merge(const RowPart* part1, int splits, int64_t n, float* lse, hipStream_t st, int tiles = 0);
 
 // ---- final_norm around the head (norm.hip) ------------------------------------
 constexpr int64_t kMaxNormD = 16384;   // hidden sizes the rms-norm kernels hold in registers
@@ -160,11 +162,32 @@ hipError_t lmhead_linear(const void* x, int64_t ldx, const void* weight, int64_t
                          hipStream_t st);
 // The projection as a teacher-logit producer: out = x[rows] . weight^T (+ addend) with,
 // when lse is not NULL, lse[t] = log-sum-exp of out's bf16 row t; rows (null: row t)
-// index nrows rows of x.  Workspace: lmhead_linear_lse_workspace_bytes.
+// index nrows rows of x.  Workspace with lse: at least linear_lse_required_bytes; with
+// lmhead_linear_lse_workspace_bytes few rows take thin.hip's kernel too.
+size_t linear_lse_required_bytes(int64_t n, int64_t v);
 size_t lmhead_linear_lse_workspace_bytes(int64_t n, int64_t v);
 hipError_t lmhead_linear_lse(const void* x, int64_t ldx, const int64_t* rows, int64_t nrows, const void* weight,
                              int64_t ldw, const void* addend, int64_t lda, void* out, int64_t ldo, float* lse,
-                             int64_t n, int64_t v, int64_t d, void* ws, hipStream_t st);
+                             int64_t n, int64_t v, int64_t d, void* ws, size_t ws_bytes, hipStream_t st);
+
+// ---- the head GEMM for few rows (thin.hip) ----------------------------------------
+constexpr int64_t kThinRows = 128;   // up to 64 rows of any vocabulary, above with vocab tiles > kThinWide
+constexpr int64_t kThinWide = 512;
+struct ThinHead {
+  const uint16_t *hidden, *weight, *markov;
+  int64_t ldh, ldw, ldm, d, v;
+  const MarkovFactors* factors;
+};
+// partials of each 128-entry half tile
+size_t thin_workspace_bytes(int64_t n, int64_t v);
+// Pass 1 of a.n <= kThinRows rows: z (one token tile of kZTile per vocab tile), z_label and the half
+// tiles' partials tpart[vocab tiles][2][n], which launch_merge turns into the bits that
+// head_kernel<STATS> and it form.
+hipError_t thin_stats(const ThinHead& x, const SlotArgs& a, const TeacherSpec& ts, const void* teacher, int tdt,
+                      int64_t ldt, float* z, float* zy, RowPart* tpart, hipStream_t st);
+// The projection of n <= kThinRows rows, and with tpart its log-sum-exp partials.
+hipError_t thin_store(const ThinHead& x, const int64_t* rows, int64_t nrows, int64_t n, void* out, int64_t ldo,
+                      RowPart* tpart, hipStream_t st);
 
 // ---- FP8 teacher head (fp8.hip) ---------------------------------------------
 size_t fp8_workspace_bytes(int64_t n, int64_t v, int64_t d);

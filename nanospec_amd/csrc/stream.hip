@@ -163,22 +163,43 @@ __global__ __launch_bounds__(kStreamThreads) void stream_stats_kernel(
 
 // One wave per row: lane l merges splits l, l + 64, .. in order, then a butterfly over the lanes
 // (symmetric: every lane ends with the same bits).  One thread per row walked up to 256 splits
-// in series: 68 us at N = 224 (256 splits), 15 us at N = 2048 (32); now 6 and 6 us.
-__device__ __forceinline__ PairState merge_row(const RowPart* __restrict__ p, int splits) {
-  PairState st = pair_init();
-  for (int s = threadIdx.x & 63; s < splits; s += 64)
-    st = pair_merge(st, PairState{p[s].mz, p[s].sz, p[s].mu, p[s].su, p[s].A});
-  return wave_reduce(st);
+// in series: 68 us at N = 224 (256 splits), 15 us at N = 2048 (32); now 7 us each.
+// With tiles > 0 a split's partial is formed here as head_kernel forms it: each vocab half's tiles of
+// the split in order, then the halves.
+__device__ __forceinline__ PairState pair_of(const RowPart& q) { return PairState{q.mz, q.sz, q.mu, q.su, q.A}; }
+__device__ __forceinline__ LseState lse_of(const RowPart& q) { return LseState{q.mz, q.sz}; }
+__device__ __forceinline__ PairState merge_of(const PairState& a, const PairState& b) { return pair_merge(a, b); }
+__device__ __forceinline__ LseState merge_of(const LseState& a, const LseState& b) { return lse_merge(a, b); }
+
+template <typename State, typename Of>
+__device__ __forceinline__ State merge_splits(const RowPart* __restrict__ part1, int64_t r, int64_t n, int splits,
+                                              int tiles, const State& init, Of&& of) {
+  State st = init;
+  for (int s = threadIdx.x & 63; s < splits; s += 64) {
+    if (tiles > 0) {
+      const int v0 = (int)((int64_t)s * tiles / splits), v1 = (int)((int64_t)(s + 1) * tiles / splits);
+      State a = init, b = init;
+      for (int j = v0; j < v1; ++j) {
+        a = merge_of(a, of(part1[(int64_t)(2 * j) * n + r]));
+        b = merge_of(b, of(part1[(int64_t)(2 * j + 1) * n + r]));
+      }
+      st = merge_of(st, merge_of(a, b));
+    } else {
+      st = merge_of(st, of(part1[r * splits + s]));
+    }
+  }
+  return st;
 }
 
 __global__ __launch_bounds__(256) void merge_kernel(const RowPart* __restrict__ part1,
                                                     const float* __restrict__ zy,
                                                     const int64_t* __restrict__ labels, int64_t v,
                                                     int splits, int64_t n, float* __restrict__ row_stats,
-                                                    TeacherSpec ts) {
+                                                    TeacherSpec ts, int tiles) {
   const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (r >= n) return;
-  const PairState st = merge_row(part1 + r * splits, splits);
+  const PairState st = wave_reduce(
+      merge_splits(part1, r, n, splits, tiles, pair_init(), [](const RowPart& q) { return pair_of(q); }));
   if ((threadIdx.x & 63) != 0) return;
   const float lz = st.mz + logf(st.sz);
   float lu = st.mu + logf(st.su);
@@ -201,33 +222,32 @@ __global__ __launch_bounds__(256) void merge_kernel(const RowPart* __restrict__ 
 }
 
 hipError_t launch_merge(const RowPart* part1, const float* zy, int64_t v, int splits, const SlotArgs& a,
-                        float* row_stats, hipStream_t st, const TeacherSpec* ts) {
+                        float* row_stats, hipStream_t st, const TeacherSpec* ts, int tiles) {
   const int64_t blocks = (a.n + 3) / 4;
   const TeacherSpec none{nullptr, 0, nullptr};
   NS_TIMED("merge_rows", st);
   if (blocks > 0)
     hipLaunchKernelGGL(merge_kernel, dim3((unsigned)blocks), dim3(256), 0, st, part1, zy, a.labels, v,
-                       splits, a.n, row_stats, ts ? *ts : none);
+                       splits, a.n, row_stats, ts ? *ts : none, tiles);
   return hipGetLastError();
 }
 
 __global__ __launch_bounds__(256) void lse_merge_kernel(const RowPart* __restrict__ part1, int splits, int64_t n,
-                                                        float* __restrict__ lse) {
+                                                        float* __restrict__ lse, int tiles) {
   const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (r >= n) return;
-  const RowPart* p = part1 + r * splits;
-  LseState st = {kNegBig, 0.f};   // as merge_row, over (mz, sz)
-  for (int s = threadIdx.x & 63; s < splits; s += 64) st = lse_merge(st, LseState{p[s].mz, p[s].sz});
+  LseState st = merge_splits(part1, r, n, splits, tiles, LseState{kNegBig, 0.f},
+                             [](const RowPart& q) { return lse_of(q); });
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) st = lse_merge(st, LseState{__shfl_xor(st.m, off), __shfl_xor(st.s, off)});
   if ((threadIdx.x & 63) == 0) lse[r] = st.m + logf(st.s);
 }
 
-hipError_t launch_lse_merge(const RowPart* part1, int splits, int64_t n, float* lse, hipStream_t st) {
+hipError_t launch_lse_merge(const RowPart* part1, int splits, int64_t n, float* lse, hipStream_t st, int tiles) {
   const int64_t blocks = (n + 3) / 4;
   NS_TIMED("lse_merge", st);
   if (blocks > 0)
-    hipLaunchKernelGGL(lse_merge_kernel, dim3((unsigned)blocks), dim3(256), 0, st, part1, splits, n, lse);
+    hipLaunchKernelGGL(lse_merge_kernel, dim3((unsigned)blocks), dim3(256), 0, st, part1, splits, n, lse, tiles);
   return hipGetLastError();
 }
 

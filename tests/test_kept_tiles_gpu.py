@@ -49,7 +49,10 @@ def _assert_same(a, b):
 
 
 @pytest.mark.parametrize("n,d,v", [(8, 64, 8), (40, 64, 264), (264, 128, 2056), (512, 192, 65536 + 136),
-                                   (136, 320, 65536)])
+                                   (136, 320, 65536),
+                                   # few rows and a large vocabulary: thin.hip's kernel for pass 1
+                                   (8, 320, 8456), (40, 64, 9000), (64, 128, 16384), (128, 192, 131336),
+                                   (96, 64, 131080)])
 @pytest.mark.parametrize("form", ["rows", "gathered", "lse", "fp32", "fp32_lse", "factored", "no_dl"])
 def test_kept_values_give_the_same_bits(gpu_lib, n, d, v, form):
     h, w, markov, u, slots = synthetic.head_inputs(n, d, v, 7000 + n, DEV, ragged=True)
@@ -91,3 +94,30 @@ def test_several_windows_of_rows(gpu_lib):
         assert abs(float(stats[r, 1] - lu)) < 1e-5 * abs(float(lu))
         p, t = (z - lz).exp(), (u[r].double() - lu).exp()
         assert float(stats[r, 4]) == pytest.approx(float(torch.minimum(p, t).sum()), rel=1e-4)
+
+
+@pytest.mark.parametrize("n", [1, 7, 32, 33, 64, 65, 100, 128])
+@pytest.mark.parametrize("v,d", [(8, 64), (8456, 320), (131336, 128)])
+def test_few_rows_projection(gpu_lib, n, v, d):
+    """The projection of up to 128 rows (thin.hip) is that of the same rows in a larger batch, bit for
+    bit, with an addend and with gathered rows (one out of range: NaN); its log-sum-exp that of the
+    stored logits."""
+    from nanospec_amd import head
+
+    g = torch.Generator(device=DEV).manual_seed(7400 + n)
+    x = torch.randn((300, d), generator=g, device=DEV).bfloat16()
+    w = (0.05 * torch.randn((v, d), generator=g, device=DEV)).bfloat16()
+    add = torch.randn((300, v), generator=g, device=DEV).bfloat16()
+    whole = head.lm_head_linear(x, w)
+    assert torch.equal(head.lm_head_linear(x[:n], w), whole[:n])
+    assert torch.equal(head.lm_head_linear(x[:n], w, add[:n]), head.lm_head_linear(x, w, add)[:n])
+    rows = torch.randint(0, 300, (n,), generator=g, device=DEV)
+    t = head.teacher_logits(x, w, rows)
+    assert torch.equal(t.logits, whole[rows])
+    want = torch.logsumexp(t.logits.double(), -1)
+    assert float(((t.lse.double() - want) / want).abs().max()) < 2e-6
+    rows[n // 2] = 300
+    t = head.teacher_logits(x, w, rows)
+    assert torch.isnan(t.logits[n // 2]).all() and torch.isnan(t.lse[n // 2])
+    keep = torch.arange(n, device=DEV) != n // 2
+    assert torch.equal(t.logits[keep], whole[rows[keep]]) and bool(torch.isfinite(t.lse[keep]).all())
