@@ -81,9 +81,9 @@ KERNEL_NAMES = [
     (r"stream_group_kernel<[^,]+, [^,]+, true>", "stream_group"),
     (r"stream_group_kernel<[^,]+, [^,]+, false>", "stream_group_accept"),
     (r"group_clear_kernel", "group_clear"),
-    # stream_emit_kernel<TZ, TU, TD, VEC, EMIT, ACCEPT>
-    (r"stream_emit_kernel<[^,]+, [^,]+, [^,]+, (?:true|false), true", "stream_emit"),
-    (r"stream_emit_kernel<[^,]+, [^,]+, [^,]+, (?:true|false), false", "stream_accept"),
+    # stream_emit_kernel<TZ, TU, TD, EMIT, ACCEPT>
+    (r"stream_emit_kernel<[^,]+, [^,]+, [^,]+, true", "stream_emit"),
+    (r"stream_emit_kernel<[^,]+, [^,]+, [^,]+, false", "stream_accept"),
     (r"lse_merge_kernel", "lse_merge"),
     (r"merge_kernel", "merge_rows"),
     (r"finalize_kernel", "finalize_metrics"),

@@ -37,6 +37,8 @@ constexpr int kStreamThreads = 256;
 // four; 16K entries moved 5.1 TB/s against 6.3.  The cap is for the pass that writes dl
 // only: the accept-only pass (no dl) runs 0.652 ms uncapped against 0.679 ms capped.
 constexpr int64_t kStatsElems = 32768;
+constexpr int64_t kStatsMinElems = 4096;
+constexpr int64_t kStatsGroups = 2048;   // eight workgroups a CU
 constexpr int kStatsMaxSplits = 64;
 constexpr int64_t kEmitElems = 3072;
 constexpr int kEmitMaxSplits = 256;
@@ -49,9 +51,14 @@ static int splits_for(int64_t v, int64_t elems, int max_splits) {
   return (int)s;
 }
 
+// Pass 1's ranges: kStatsElems entries, shorter (down to kStatsMinElems) where the rows alone
+// leave CUs without workgroups: N = 224, V = 50,001 (fp32) ran 448 workgroups, 42 us with element loads, now
+// 2912 with vectors 20 us.
 int stream_splits(int64_t n, int64_t v) {
-  (void)n;
-  return splits_for(v, kStatsElems, kStatsMaxSplits);
+  const int64_t want = n > 0 ? (kStatsGroups + n - 1) / n : 1;
+  int64_t elems = want > 0 ? v / want : v;
+  elems = elems < kStatsMinElems ? kStatsMinElems : elems > kStatsElems ? kStatsElems : elems;
+  return splits_for(v, elems, kStatsMaxSplits);
 }
 
 static int emit_splits(int64_t v) { return splits_for(v, kEmitElems, kEmitMaxSplits); }
@@ -108,7 +115,7 @@ __device__ __forceinline__ float block_sum(float x) {
 
 // ---------------------------------------------------------------- pass 1
 
-template <typename TZ, typename TU, bool VEC>
+template <typename TZ, typename TU>
 __global__ __launch_bounds__(kStreamThreads) void stream_stats_kernel(
     const TZ* __restrict__ z, int64_t ldz, const TU* __restrict__ u, int64_t ldu, int64_t v,
     int64_t chunk, int splits, const int64_t* __restrict__ labels, RowPart* __restrict__ part1,
@@ -119,9 +126,11 @@ __global__ __launch_bounds__(kStreamThreads) void stream_stats_kernel(
   const int64_t hi = lo + chunk < v ? lo + chunk : v;
   const TZ* zr = z + r * ldz;
   const TU* ur = u + r * ldu;
+  // 16-byte vectors whatever the rows' alignment (an odd V leaves them aligned to an element only:
+  // read one element a thread and folded one by one they took twice the time)
   PairState st = pair_init();
   int64_t scalar_from = lo;
-  if (VEC && lo < hi) {
+  if (lo < hi) {
     const int64_t nvec = (hi - lo) >> 3;
     const TZ* zb = zr + lo;
     const TU* ub = ur + lo;
@@ -138,8 +147,8 @@ __global__ __launch_bounds__(kStreamThreads) void stream_stats_kernel(
     }
     if (j < nvec) {
       float zf[8], uf[8];
-      load8(zb + j * 8, zf);
-      load8(ub + j * 8, uf);
+      load8_nt(zb + j * 8, zf);
+      load8_nt(ub + j * 8, uf);
       pair_update<8>(st, zf, uf);
     }
     scalar_from = lo + nvec * 8;
@@ -253,7 +262,7 @@ hipError_t launch_lse_merge(const RowPart* part1, int splits, int64_t n, float* 
 
 // ---------------------------------------------------------------- pass 2
 
-template <typename TZ, typename TU, typename TD, bool VEC, bool EMIT, bool ACCEPT>
+template <typename TZ, typename TU, typename TD, bool EMIT, bool ACCEPT>
 __global__ __launch_bounds__(kStreamThreads) void stream_emit_kernel(
     const TZ* __restrict__ z, int64_t ldz, const TU* __restrict__ u, int64_t ldu, int64_t v,
     int64_t chunk, int splits, const float* __restrict__ row_stats, const int64_t* __restrict__ labels,
@@ -274,7 +283,7 @@ __global__ __launch_bounds__(kStreamThreads) void stream_emit_kernel(
   const float cp = y == kIgnoreIndex ? w * c_kl : w * (c_ce + c_kl), ct = w * c_kl, cy = w * c_ce;
   float acc = 0.f;
   int64_t scalar_from = lo;
-  if (VEC && lo < hi) {
+  if (lo < hi) {
     const int64_t nvec = (hi - lo) >> 3;
     // U groups of 8 per iteration: all 2U loads are issued before any is used
     auto body = [&](auto uc, int64_t j) {
@@ -824,17 +833,11 @@ static hipError_t stats_dispatch(const void* z, int64_t ldz, const void* u, int6
                                  const SlotArgs& a, const StreamWs& w, int S, hipStream_t st) {
   const TZ* zp = static_cast<const TZ*>(z);
   const TU* up = static_cast<const TU*>(u);
-  const bool vec = aligned16(z) && aligned16(u) && (ldz * (int64_t)sizeof(TZ)) % 16 == 0 &&
-                   (ldu * (int64_t)sizeof(TU)) % 16 == 0;
   const int64_t chunk = split_chunk(v, S);
   dim3 grid((unsigned)(S * a.n));
   NS_TIMED("stream_stats", st);
-  if (vec)
-    hipLaunchKernelGGL((stream_stats_kernel<TZ, TU, true>), grid, dim3(kStreamThreads), 0, st, zp, ldz, up,
-                       ldu, v, chunk, S, a.labels, w.part1, w.zy);
-  else
-    hipLaunchKernelGGL((stream_stats_kernel<TZ, TU, false>), grid, dim3(kStreamThreads), 0, st, zp, ldz,
-                       up, ldu, v, chunk, S, a.labels, w.part1, w.zy);
+  hipLaunchKernelGGL((stream_stats_kernel<TZ, TU>), grid, dim3(kStreamThreads), 0, st, zp, ldz, up, ldu, v, chunk, S,
+                     a.labels, w.part1, w.zy);
   return hipGetLastError();
 }
 
@@ -845,20 +848,12 @@ static hipError_t emit_dispatch(const void* z, int64_t ldz, const void* u, int64
   const TZ* zp = static_cast<const TZ*>(z);
   const TU* up = static_cast<const TU*>(u);
   TZ* dp = static_cast<TZ*>(dl);  // dl has the logits dtype (objective.py:80)
-  bool vec = aligned16(z) && aligned16(u) && (ldz * (int64_t)sizeof(TZ)) % 16 == 0 &&
-             (ldu * (int64_t)sizeof(TU)) % 16 == 0;
-  if (EMIT) vec = vec && aligned16(dl) && (ldd * (int64_t)sizeof(TZ)) % 16 == 0;
   const int64_t chunk = split_chunk(v, S);
   dim3 grid((unsigned)(S * a.n));
   NS_TIMED(EMIT ? "stream_emit" : "stream_accept", st);
-  if (vec)
-    hipLaunchKernelGGL((stream_emit_kernel<TZ, TU, TZ, true, EMIT, ACCEPT>), grid, dim3(kStreamThreads), EMIT ? kEmitLds : 0,
-                       st, zp, ldz, up, ldu, v, chunk, S, row_stats, a.labels, a.weights, a.c_ce, a.c_kl,
-                       a.inv_acc, dp, ldd, parta);
-  else
-    hipLaunchKernelGGL((stream_emit_kernel<TZ, TU, TZ, false, EMIT, ACCEPT>), grid, dim3(kStreamThreads), EMIT ? kEmitLds : 0,
-                       st, zp, ldz, up, ldu, v, chunk, S, row_stats, a.labels, a.weights, a.c_ce, a.c_kl,
-                       a.inv_acc, dp, ldd, parta);
+  hipLaunchKernelGGL((stream_emit_kernel<TZ, TU, TZ, EMIT, ACCEPT>), grid, dim3(kStreamThreads), EMIT ? kEmitLds : 0,
+                     st, zp, ldz, up, ldu, v, chunk, S, row_stats, a.labels, a.weights, a.c_ce, a.c_kl, a.inv_acc, dp,
+                     ldd, parta);
   return hipGetLastError();
 }
 
