@@ -173,43 +173,73 @@ __global__ __launch_bounds__(kStreamThreads) void stream_stats_kernel(
 // One wave per row: lane l merges splits l, l + 64, .. in order, then a butterfly over the lanes
 // (symmetric: every lane ends with the same bits).  One thread per row walked up to 256 splits
 // in series: 68 us at N = 224 (256 splits), 15 us at N = 2048 (32); now 7 us each.
-// With tiles > 0 a split's partial is formed here as head_kernel forms it: each vocab half's tiles of
-// the split in order, then the halves.
+//
+// With TILES the partials are those of half vocab tiles (thin.hip): a workgroup per row, thread s
+// first forms split s's partial as head_kernel does (each vocab half's tiles in order, then the
+// halves), then the first wave merges the splits as above.  (One wave walking all of a row's tiles
+// took 19 us at n = 8, 970 tiles.)
 __device__ __forceinline__ PairState pair_of(const RowPart& q) { return PairState{q.mz, q.sz, q.mu, q.su, q.A}; }
 __device__ __forceinline__ LseState lse_of(const RowPart& q) { return LseState{q.mz, q.sz}; }
 __device__ __forceinline__ PairState merge_of(const PairState& a, const PairState& b) { return pair_merge(a, b); }
 __device__ __forceinline__ LseState merge_of(const LseState& a, const LseState& b) { return lse_merge(a, b); }
-
-template <typename State, typename Of>
-__device__ __forceinline__ State merge_splits(const RowPart* __restrict__ part1, int64_t r, int64_t n, int splits,
-                                              int tiles, const State& init, Of&& of) {
-  State st = init;
-  for (int s = threadIdx.x & 63; s < splits; s += 64) {
-    if (tiles > 0) {
-      const int v0 = (int)((int64_t)s * tiles / splits), v1 = (int)((int64_t)(s + 1) * tiles / splits);
-      State a = init, b = init;
-      for (int j = v0; j < v1; ++j) {
-        a = merge_of(a, of(part1[(int64_t)(2 * j) * n + r]));
-        b = merge_of(b, of(part1[(int64_t)(2 * j + 1) * n + r]));
-      }
-      st = merge_of(st, merge_of(a, b));
-    } else {
-      st = merge_of(st, of(part1[r * splits + s]));
-    }
-  }
-  return st;
+__device__ __forceinline__ LseState wave_reduce(LseState s) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) s = lse_merge(s, LseState{__shfl_xor(s.m, off), __shfl_xor(s.s, off)});
+  return s;
 }
 
+// The row's state, for lane 0 of a wave of row r; the other threads of a TILES workgroup leave with
+// r = -1.
+template <bool TILES, typename State, typename Of>
+__device__ __forceinline__ State merge_row(const RowPart* __restrict__ part1, int64_t n, int splits, int tiles,
+                                           const State& init, Of&& of, int64_t& r) {
+  if constexpr (TILES) {
+    __shared__ State sh[256];
+    r = blockIdx.x;
+    for (int s0 = 0; s0 < splits; s0 += 256) {   // (splits <= 256)
+      const int s = s0 + (int)threadIdx.x;
+      if (s < splits) {
+        const int v0 = (int)((int64_t)s * tiles / splits), v1 = (int)((int64_t)(s + 1) * tiles / splits);
+        State a = init, b = init;
+        for (int j = v0; j < v1; ++j) {
+          const RowPart qa = part1[(int64_t)(2 * j) * n + r], qb = part1[(int64_t)(2 * j + 1) * n + r];
+          a = merge_of(a, of(qa));
+          b = merge_of(b, of(qb));
+        }
+        sh[s] = merge_of(a, b);
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) {
+      r = -1;
+      return init;
+    }
+    State st = init;
+    for (int s = threadIdx.x; s < splits; s += 64) st = merge_of(st, sh[s]);
+    return wave_reduce(st);
+  } else {
+    r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    State st = init;
+    if (r >= n) {
+      r = -1;
+      return st;
+    }
+    const RowPart* p = part1 + r * splits;
+    for (int s = threadIdx.x & 63; s < splits; s += 64) st = merge_of(st, of(p[s]));
+    return wave_reduce(st);
+  }
+}
+
+template <bool TILES>
 __global__ __launch_bounds__(256) void merge_kernel(const RowPart* __restrict__ part1,
                                                     const float* __restrict__ zy,
                                                     const int64_t* __restrict__ labels, int64_t v,
                                                     int splits, int64_t n, float* __restrict__ row_stats,
                                                     TeacherSpec ts, int tiles) {
-  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (r >= n) return;
-  const PairState st = wave_reduce(
-      merge_splits(part1, r, n, splits, tiles, pair_init(), [](const RowPart& q) { return pair_of(q); }));
-  if ((threadIdx.x & 63) != 0) return;
+  int64_t r;
+  const PairState st = merge_row<TILES>(part1, n, splits, tiles, pair_init(),
+                                        [](const RowPart& q) { return pair_of(q); }, r);
+  if (r < 0 || (threadIdx.x & 63) != 0) return;
   const float lz = st.mz + logf(st.sz);
   float lu = st.mu + logf(st.su);
   if (ts.lse) {   // the teacher's producer formed its log-normaliser; KL follows pass 2
@@ -232,31 +262,30 @@ __global__ __launch_bounds__(256) void merge_kernel(const RowPart* __restrict__ 
 
 hipError_t launch_merge(const RowPart* part1, const float* zy, int64_t v, int splits, const SlotArgs& a,
                         float* row_stats, hipStream_t st, const TeacherSpec* ts, int tiles) {
-  const int64_t blocks = (a.n + 3) / 4;
+  const int64_t blocks = tiles > 0 ? a.n : (a.n + 3) / 4;
   const TeacherSpec none{nullptr, 0, nullptr};
   NS_TIMED("merge_rows", st);
   if (blocks > 0)
-    hipLaunchKernelGGL(merge_kernel, dim3((unsigned)blocks), dim3(256), 0, st, part1, zy, a.labels, v,
-                       splits, a.n, row_stats, ts ? *ts : none, tiles);
+    hipLaunchKernelGGL(tiles > 0 ? merge_kernel<true> : merge_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, st,
+                       part1, zy, a.labels, v, splits, a.n, row_stats, ts ? *ts : none, tiles);
   return hipGetLastError();
 }
 
+template <bool TILES>
 __global__ __launch_bounds__(256) void lse_merge_kernel(const RowPart* __restrict__ part1, int splits, int64_t n,
                                                         float* __restrict__ lse, int tiles) {
-  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (r >= n) return;
-  LseState st = merge_splits(part1, r, n, splits, tiles, LseState{kNegBig, 0.f},
-                             [](const RowPart& q) { return lse_of(q); });
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) st = lse_merge(st, LseState{__shfl_xor(st.m, off), __shfl_xor(st.s, off)});
-  if ((threadIdx.x & 63) == 0) lse[r] = st.m + logf(st.s);
+  int64_t r;
+  const LseState st = merge_row<TILES>(part1, n, splits, tiles, LseState{kNegBig, 0.f},
+                                       [](const RowPart& q) { return lse_of(q); }, r);
+  if (r >= 0 && (threadIdx.x & 63) == 0) lse[r] = st.m + logf(st.s);
 }
 
 hipError_t launch_lse_merge(const RowPart* part1, int splits, int64_t n, float* lse, hipStream_t st, int tiles) {
-  const int64_t blocks = (n + 3) / 4;
+  const int64_t blocks = tiles > 0 ? n : (n + 3) / 4;
   NS_TIMED("lse_merge", st);
   if (blocks > 0)
-    hipLaunchKernelGGL(lse_merge_kernel, dim3((unsigned)blocks), dim3(256), 0, st, part1, splits, n, lse, tiles);
+    hipLaunchKernelGGL(tiles > 0 ? lse_merge_kernel<true> : lse_merge_kernel<false>, dim3((unsigned)blocks),
+                       dim3(256), 0, st, part1, splits, n, lse, tiles);
   return hipGetLastError();
 }
 

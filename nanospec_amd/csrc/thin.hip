@@ -123,6 +123,12 @@ __global__ __launch_bounds__(64 * W) void thin_kernel(ThinParams p) {
   const bool none = vb >= p.v;
   const bool full = vb + 128 <= p.v;
 
+  // Rows whose pitch is a multiple of 4 KB meet the same memory channels while all workgroups walk K
+  // in step: an XCD's workgroups start up to 7 us apart then (d = 2048, V = 248,320: n = 8 249 -> 225
+  // us, 56 262 -> 243, 120 289 -> 269; at d = 4096 and other pitches it changed nothing).
+  if (p.ldw % 2048 == 0)
+    for (int q = (int)(blockIdx.x / kNumXcd) % 8; q > 0; --q) __builtin_amdgcn_s_sleep(32);
+
   f32x16_t acc[4][NB];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
