@@ -168,7 +168,8 @@ def check(status: int, name: str) -> None:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else _c.c_void_p(t.data_ptr())
+    # a plain int (the argtypes make it a void*): a c_void_p object per operand cost 0.4 us each
+    return None if t is None else t.data_ptr()
 
 
 def dtype_code(t: torch.Tensor) -> int:
@@ -180,8 +181,10 @@ def dtype_code(t: torch.Tensor) -> int:
 
 
 def stream(device: torch.device):
-    """hipStream_t of torch's current stream on ``device``."""
-    return _c.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """hipStream_t of torch's current stream on ``device`` (the raw handle: building the Stream object
+    takes 3 us)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def require_device(*tensors: torch.Tensor) -> torch.device:
@@ -206,11 +209,12 @@ def workspace(kind: int, n: int, v: int, d: int, device: torch.device) -> torch.
 
 def rows_2d(t: torch.Tensor, cols: int) -> tuple[torch.Tensor, int]:
     """View ``t`` as [rows, cols] with unit column stride; returns (view, ld)."""
-    t2 = t.reshape(-1, cols)
-    if t2.stride(-1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < cols):
+    t2 = t if t.dim() == 2 and t.shape[1] == cols else t.reshape(-1, cols)
+    rows, (ld, step) = t2.shape[0], t2.stride()
+    if step != 1 or (rows > 1 and ld < cols):
         t2 = t2.contiguous()
-    ld = t2.stride(0) if t2.shape[0] > 1 else cols
-    return t2, ld
+        ld = t2.stride(0)
+    return t2, ld if rows > 1 else cols
 
 
 def copy_rows(src: torch.Tensor, rows_map: torch.Tensor, n_dst: int, out: torch.Tensor) -> torch.Tensor:

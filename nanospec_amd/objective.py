@@ -83,10 +83,15 @@ def _slot_inputs(prepared, n: int, device: torch.device):
             f"{tuple(weights.shape)}, target_ids {tuple(labels.shape)}, valid {tuple(valid.shape)}"
         )
     k = weights.shape[-1] if weights.dim() > 0 else 1
-    w = weights.reshape(-1).to(device=device, dtype=torch.float32).contiguous()
-    y = labels.reshape(-1).to(device=device, dtype=torch.int64).contiguous()
-    v = valid.reshape(-1).to(device=device, dtype=torch.bool).contiguous()
-    return w, y, v.view(torch.uint8), k
+    return (_flat(weights, torch.float32, device), _flat(labels, torch.int64, device),
+            _flat(valid, torch.bool, device), k)
+
+
+def _flat(t: torch.Tensor, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
+    """[N] contiguous view or copy of ``t`` in ``dtype`` on ``device``."""
+    if t.dtype != dtype or t.device != device:
+        t = t.to(device=device, dtype=dtype)
+    return t.contiguous().view(-1)
 
 
 @torch.no_grad()
