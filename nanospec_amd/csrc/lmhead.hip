@@ -1320,13 +1320,13 @@ struct HeadPlan {
   int xa, xb;  // XCD round block (wg_coords): token tiles x splits, 0 = unblocked
 };
 
-
 HeadPlan head_plan(int64_t n, int64_t v) {
   HeadPlan pl;
   pl.tt = (int)((n + BN - 1) / BN);
   pl.vt = (int)((v + BM - 1) / BM);
   // both operands stage 256 rows x 64 bf16 per K step, so the block only counts tiles
-  const SplitPlan sp = split_plan(pl.tt, pl.vt, device_cus());
+  const int cus = device_cus();
+  const SplitPlan sp = split_plan(pl.tt, pl.vt, cus < kMaxHeadSplits ? cus : kMaxHeadSplits);
   pl.splits = sp.splits;
   pl.grid = pl.tt * sp.splits;
   pl.xa = sp.xa;

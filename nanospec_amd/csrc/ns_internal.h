@@ -41,10 +41,13 @@ struct TeacherSpec {
   int64_t nt;
   const float* lse;
 };
+// Vocab splits of a head plan at most (one a CU): a row merge over half tiles forms each split's state
+// in a thread of its own.
+constexpr int kMaxHeadSplits = 256;
 // Merge first-pass partials part1[N][S] (+ z_y[N]) into row_stats (lse_z, lse_u, ce, kl, z_y).
 // With ts (its lse given) lse_u comes from ts and KL is left to the finalize.  tiles > 0: part1
 // holds the partials of half vocab tiles instead, [tiles][2][N], of which each of S splits takes a
-// contiguous range.
+// contiguous range (S <= kMaxHeadSplits).
 hipError_t launch_merge(const RowPart* part1, const float* zy, int64_t v, int splits, const SlotArgs& a,
                         float* row_stats, hipStream_t st, const TeacherSpec* ts = nullptr, int tiles = 0);
 // Sum accept partials parta[N][S], form block lengths and the six metrics; with partk

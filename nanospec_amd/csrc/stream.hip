@@ -194,20 +194,17 @@ template <bool TILES, typename State, typename Of>
 __device__ __forceinline__ State merge_row(const RowPart* __restrict__ part1, int64_t n, int splits, int tiles,
                                            const State& init, Of&& of, int64_t& r) {
   if constexpr (TILES) {
-    __shared__ State sh[256];
+    __shared__ State sh[kMaxHeadSplits];   // as many as the workgroup's threads
     r = blockIdx.x;
-    for (int s0 = 0; s0 < splits; s0 += 256) {   // (splits <= 256)
-      const int s = s0 + (int)threadIdx.x;
-      if (s < splits) {
-        const int v0 = (int)((int64_t)s * tiles / splits), v1 = (int)((int64_t)(s + 1) * tiles / splits);
-        State a = init, b = init;
-        for (int j = v0; j < v1; ++j) {
-          const RowPart qa = part1[(int64_t)(2 * j) * n + r], qb = part1[(int64_t)(2 * j + 1) * n + r];
-          a = merge_of(a, of(qa));
-          b = merge_of(b, of(qb));
-        }
-        sh[s] = merge_of(a, b);
+    if (const int s = (int)threadIdx.x; s < splits) {
+      const int v0 = (int)((int64_t)s * tiles / splits), v1 = (int)((int64_t)(s + 1) * tiles / splits);
+      State a = init, b = init;
+      for (int j = v0; j < v1; ++j) {
+        const RowPart qa = part1[(int64_t)(2 * j) * n + r], qb = part1[(int64_t)(2 * j + 1) * n + r];
+        a = merge_of(a, of(qa));
+        b = merge_of(b, of(qb));
       }
+      sh[s] = merge_of(a, b);
     }
     __syncthreads();
     if (threadIdx.x >= 64) {
@@ -262,6 +259,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const RowPart* __restrict__ 
 
 hipError_t launch_merge(const RowPart* part1, const float* zy, int64_t v, int splits, const SlotArgs& a,
                         float* row_stats, hipStream_t st, const TeacherSpec* ts, int tiles) {
+  if (tiles > 0 && splits > kMaxHeadSplits) return hipErrorInvalidValue;
   const int64_t blocks = tiles > 0 ? a.n : (a.n + 3) / 4;
   const TeacherSpec none{nullptr, 0, nullptr};
   NS_TIMED("merge_rows", st);
@@ -281,6 +279,7 @@ __global__ __launch_bounds__(256) void lse_merge_kernel(const RowPart* __restric
 }
 
 hipError_t launch_lse_merge(const RowPart* part1, int splits, int64_t n, float* lse, hipStream_t st, int tiles) {
+  if (tiles > 0 && splits > kMaxHeadSplits) return hipErrorInvalidValue;
   const int64_t blocks = tiles > 0 ? n : (n + 3) / 4;
   NS_TIMED("lse_merge", st);
   if (blocks > 0)
