@@ -1420,15 +1420,46 @@ struct BwdPlan {
   int xa, xb;        // XCD block (dh_kernel's tile order), 0 = unblocked
 };
 
-// K splits of the dh GEMM: of the counts that fill 1, 2, .. kMaxRounds rounds of the CUs, the one
-// of least cost in units of a K entry of one 256 x 256 tile (24 ns: 0.77 us a 32-K stage):
-// rounds x (a workgroup's share of K + kTileCost for its first fills and its partial tile's
-// store, about 15 us) + the partials' sum (4 bytes per entry and split at 4.5 TB/s).  (ceil of
-// four rounds, at most 16 splits, gave N = 1001, d = 5120, V = 248,320 13 splits, 4.06 rounds:
-// 2.34 ms, with 16 1.89; N = 224 16 splits, 1.25 rounds: 0.77 ms, with 12 0.64; N = 64, d = 256
-// 16 workgroups.)
-constexpr int kMaxRounds = 6;
-constexpr double kTileCost = 640, kPartialCost = 3.7e-5;
+// K splits of the dh GEMM: of the counts that fill part of a round of the CUs (down to a quarter), or
+// 1, 2, .. kMaxRounds whole ones, and the largest the sum takes in four groups (kFourGroups), the one of
+// least cost in units of a K entry of one 256 x 256 tile (24 ns: 0.77 us a 32-K stage): rounds x (a
+// workgroup's share of K + kTileCost for its first fills and its partial tile's store, about 15 us)
+// + the partials' write and sum (8 bytes per entry and split at 5.6 TB/s) + kSplitCost a split (0.1 us,
+// the sum's chain) + kGroupsCost (2.4 us) past four groups, where a norm that follows needs a launch more.
+// Counts whose workgroups are not a multiple of the XCDs are rounded down to one: such a grid is not
+// laid out by XCD (N = 700, d = 1024, V = 32,000: 12 tiles x 20 splits 59 us, x 21 84 us).
+//
+// Against at most 16 splits for four rounds (dh in us): V = 248,320, d = 5120: N = 224 12 splits 596
+// for 764, N = 700 4 splits 1496 for 1649; V = 32,000, d = 1024: N = 8 24 for 41; V = 8192, d = 2048: N
+// = 1000 49 for 72.  Against whole rounds only (V = 4096): d = 256, N = 224 64 splits 23.3, 24 splits
+// 20.1; d = 1024, N = 64 64 splits 22.3, 24 splits 18.7.
+constexpr int kMaxRounds = 6, kFourGroups = 24;
+constexpr double kTileCost = 640, kPartialCost = 6e-5, kSplitCost = 4, kGroupsCost = 100;
+
+int bwd_splits(int64_t n, int64_t v, int64_t d, int tiles, int kt_total, int cus) {
+  int step = 1;   // splits whose workgroups are a multiple of the XCDs
+  while ((int64_t)tiles * step % kNumXcd) step *= 2;
+  int ks = 0, last = 0;
+  double best = 0;
+  const double per_split = (double)n * d * kPartialCost + kSplitCost;
+  auto consider = [&](int64_t x) {
+    int c = x < 1 ? 1 : x > kt_total ? kt_total : (int)x;
+    if (c >= step) c &= ~(step - 1);
+    if (c == last) return;
+    last = c;
+    const double cost = (double)(((int64_t)tiles * c + cus - 1) / cus) * ((double)v / c + kTileCost) + c * per_split +
+                        (c > kFourGroups ? kGroupsCost : 0);
+    if (ks == 0 || cost < best || (cost == best && c < ks)) {
+      best = cost;
+      ks = c;
+    }
+  };
+  for (int eighths : {2, 3, 4, 6}) consider(eighths * cus / 8 / tiles);
+  if (tiles <= kMaxRounds * cus / kFourGroups) consider(kFourGroups);
+  // (more rounds share the work no more evenly than one that is full)
+  for (int j = 1; j <= (cus % tiles ? kMaxRounds : 1); ++j) consider(j * cus / tiles);
+  return ks;
+}
 
 BwdPlan bwd_plan(int64_t n, int64_t v, int64_t d, int64_t r = 0) {
   BwdPlan pl;
@@ -1438,21 +1469,7 @@ BwdPlan bwd_plan(int64_t n, int64_t v, int64_t d, int64_t r = 0) {
   pl.kt_total = (int)((v + BK - 1) / BK);
   const int tiles = pl.mt * pl.ct;
   const int cus = device_cus();
-  int ks = 1;   // no tiles: nothing launches
-  if (tiles > 0) {
-    double best = 0;
-    for (int j = 1; j <= kMaxRounds; ++j) {
-      int c = (int)((int64_t)j * cus / tiles);
-      if (c < 1) c = 1;
-      if (c > pl.kt_total) c = pl.kt_total;
-      const double cost = ((int64_t)tiles * c + cus - 1) / cus * ((double)v / c + kTileCost) +
-                          (double)c * n * d * kPartialCost;
-      if (j == 1 || cost < best) {
-        best = cost;
-        ks = c;
-      }
-    }
-  }
+  const int ks = tiles > 0 ? bwd_splits(n, v, d, tiles, pl.kt_total, cus) : 1;   // no tiles: nothing launches
   pl.ksplit = ks;
   pl.grid_main = tiles * ks;
   // Markov tiles run after the dh tiles as one extra round: enough K splits to give

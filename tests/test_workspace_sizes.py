@@ -22,3 +22,18 @@ def test_few_rows_have_at_most_256_vocab_splits(lib, v):
         tiles = up((v + 255) // 256 * 2 * n * ROW_PART)
         parts = lib.ns_workspace_bytes(_lib.NS_WS_TEACHER_LOGITS, n, v, 0) - tiles
         assert 0 < parts <= up(n * 256 * ROW_PART)
+
+
+@pytest.mark.parametrize("v,d", [(4096, 256), (4096, 2048), (32000, 1024), (65536, 256), (248320, 2048),
+                                 (248320, 5120)])
+@pytest.mark.parametrize("n", [1, 64, 224, 300, 500, 700, 1001, 1500, 4096])
+def test_dh_splits_fill_the_xcds_evenly(lib, n, v, d):
+    """dh's grid is laid out by XCD only when its workgroups are a multiple of the 8 XCDs: no plan
+    leaves it short of that (the workspace is its splits' fp32 partials), and no small vocabulary is cut
+    into shares that cost more to sum than they save."""
+    tiles = -(-n // 256) * -(-d // 256)
+    splits = lib.ns_workspace_bytes(_lib.NS_WS_LMHEAD_BWD, n, v, d) // (4 * n * d)
+    assert 1 <= splits <= -(-v // 64)
+    assert splits * tiles % 8 == 0 or splits < 8
+    if v <= 4096:
+        assert splits <= 24
