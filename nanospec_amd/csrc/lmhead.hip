@@ -1242,9 +1242,10 @@ void dh_kernel(BwdParams p) {
 // contiguous share of the splits in order, then the groups' sums are added in order.  One
 // thread walking 64 splits took 33 us for N = 224, d = 256 (56 workgroups, one load after the
 // other); with 16 groups 7 us.
+// `out` may be the first split's partial itself (ldo = d): what a workgroup stores only it has read.
 template <int G, typename OUT>
-__global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restrict__ part, int ksplit, int64_t n,
-                                                           int64_t d, OUT* __restrict__ out, int64_t ldo) {
+__global__ __launch_bounds__(256) void sum_partials_kernel(const float* part, int ksplit, int64_t n, int64_t d,
+                                                           OUT* out, int64_t ldo) {
   constexpr int Q = 256 / G;   // float4 columns per workgroup
   const int g = G > 1 ? threadIdx.x / Q : 0, q = threadIdx.x % Q;
   const int64_t idx = ((int64_t)blockIdx.x * Q + q) * 4;
@@ -1822,7 +1823,18 @@ hipError_t lmhead_backward_ext(const void* dl, int64_t ldd, const void* weight, 
     if (e != hipSuccess) return e;
   }
   if (norm) {
-    hipError_t e = rms_norm_backward_rows(p.part, pl.ksplit, nullptr, 0, *norm, dh, lddh, n, d, norm_ws, st);
+    // The norm's backward takes a row a workgroup and adds the splits of a column in one thread: 16
+    // groups of them one after the other cost more than the GEMM had gained (d = 256, whole call:
+    // V = 32,000, N = 8 53 us, N = 224 63 us; V = 248,320, N = 8 73 us).  Past four groups they are
+    // summed first, in the same order and where the first partial lies: 30, 34 and 39 us.  With four
+    // groups a launch more is no gain (V = 4096, d = 5120, N = 224, 12 splits: 42.1 against 43.1 us).
+    int ksplit = pl.ksplit;
+    if (split_groups(ksplit) > 4) {
+      NS_TIMED("dh_reduce", st);
+      if (const hipError_t e = launch_sum_partials(p.part, ksplit, n, d, p.part, d, st); e != hipSuccess) return e;
+      ksplit = 1;
+    }
+    hipError_t e = rms_norm_backward_rows(p.part, ksplit, nullptr, 0, *norm, dh, lddh, n, d, norm_ws, st);
     if (e != hipSuccess) return e;
   } else {
     NS_TIMED("dh_reduce", st);

@@ -91,6 +91,26 @@ def test_fused_norm_backward_equals_unfused(gpu_lib, n, v, d):
     assert torch.equal(dx1, dx2) and torch.equal(wg1, wg2)
 
 
+@pytest.mark.parametrize("n,v,d", [
+    (1, 8192, 64), (8, 8192, 256), (64, 4096, 1024),     # a tile of d whose K is split over most of the CUs
+    (224, 8192, 256), (257, 4096, 264), (1000, 32000, 256),
+    (224, 4096, 2048), (224, 8192, 5120), (8, 64, 64),   # one to four groups of splits; a single split
+])
+def test_fused_norm_backward_over_split_counts(gpu_lib, n, v, d):
+    """The splits' partials summed inside the norm's backward, or before it, are dh's own sum: the same
+    bits as dh, then the norm's backward."""
+    x, w, g = _norm_inputs(n, d, 300 + n)
+    _, saved = ops.rms_norm(x, w, EPS)
+    dl = (1e-3 * torch.randn((n, v), generator=g, device=DEV)).bfloat16()
+    wlm = (0.02 * torch.randn((v, d), generator=g, device=DEV)).bfloat16()
+    wg1 = torch.empty(d, dtype=torch.bfloat16, device=DEV)
+    wg2 = torch.empty_like(wg1)
+    dx1 = head.lm_head_norm_backward(dl, wlm, (saved, w, wg1))
+    dx2 = ops.rms_norm_backward(head.lm_head_linear_backward(dl, wlm), saved, w, wg2)
+    torch.cuda.synchronize()
+    assert torch.equal(dx1, dx2) and torch.equal(wg1, wg2)
+
+
 def test_markov_backward_with_norm_equals_unfused(gpu_lib):
     n, v, d, r = 512, 4096, 320, 64
     x, w, g = _norm_inputs(n, d, 5)
