@@ -42,7 +42,17 @@ struct ThinParams {
   int64_t ldo;
   RowPart* tpart;           // [vt][2][n] partials of each half tile (STORE: or null)
   int vt;
+  bool stagger;
 };
+
+// Weight rows whose pitch is a multiple of 4 KB meet the same memory channels while all workgroups walk
+// K in step.  Where W comes from memory the workgroups of an XCD then start apart: projections in us
+// together / apart, n = 8 and 56: V = 248,320, d = 2048 255 / 231, 268 / 246; V = 65,536, d = 4096 127 /
+// 116, 131 / 122; V = 98,304, d = 2048 (384 MB) 83 / 81, 110 / 108; V = 40,960, d = 4096 (320 MB) 71 / 67,
+// 74 / 74.  A smaller W is held by the Infinity Cache (256 MB) and the delay is a tail: V = 65,536, d =
+// 2048 41 / 42, 43 / 47; V = 32,768 22 / 27, 33 / 38; V = 8192 20 / 23, 32 / 35.  (n = 120: unchanged
+// below 700 MB, 288 / 268 at V = 248,320.)
+constexpr int64_t kStaggerBytes = int64_t(5) << 26;
 
 // LDS of a workgroup of W waves: each wave's own two stages of its 128 weight rows (64 K entries,
 // 128 bytes a row, lds_off's swizzle), then the stages of the NB x 32 hidden rows they share: three,
@@ -123,10 +133,8 @@ __global__ __launch_bounds__(64 * W) void thin_kernel(ThinParams p) {
   const bool none = vb >= p.v;
   const bool full = vb + 128 <= p.v;
 
-  // Rows whose pitch is a multiple of 4 KB meet the same memory channels while all workgroups walk K
-  // in step: an XCD's workgroups start up to 7 us apart then (d = 2048, V = 248,320: n = 8 249 -> 225
-  // us, 56 262 -> 243, 120 289 -> 269; at d = 4096 and other pitches it changed nothing).
-  if (p.ldw % 2048 == 0)
+  // an XCD's workgroups start up to 7 us apart (kStaggerBytes)
+  if (p.stagger)
     for (int q = (int)(blockIdx.x / kNumXcd) % 8; q > 0; --q) __builtin_amdgcn_s_sleep(32);
 
   f32x16_t acc[4][NB];
@@ -315,8 +323,10 @@ __global__ __launch_bounds__(64 * W) void thin_kernel(ThinParams p) {
 }
 
 template <int MODE, typename TT, bool LSE>
-hipError_t launch_thin(const ThinParams& p, const char* name, hipStream_t st) {
+hipError_t launch_thin(const ThinParams& args, const char* name, hipStream_t st) {
   NS_TIMED(name, st);
+  ThinParams p = args;
+  p.stagger = p.ldw % 2048 == 0 && p.v * p.d * 2 >= kStaggerBytes;
   // 512 vocab rows a workgroup, or 256 where those would leave CUs without one
   const bool wide = p.vt > kThinWide;
   const dim3 grid((unsigned)(wide ? (p.vt + 1) / 2 : p.vt));

@@ -121,3 +121,16 @@ def test_few_rows_projection(gpu_lib, n, v, d):
     assert torch.isnan(t.logits[n // 2]).all() and torch.isnan(t.lse[n // 2])
     keep = torch.arange(n, device=DEV) != n // 2
     assert torch.equal(t.logits[keep], whole[rows[keep]]) and bool(torch.isfinite(t.lse[keep]).all())
+
+
+@pytest.mark.parametrize("v", [81912, 81920, 84008])   # d = 2048: below, at and past 320 MiB of W
+@pytest.mark.parametrize("n", [8, 64])
+def test_few_rows_with_workgroups_started_apart(gpu_lib, n, v):
+    """Whether the workgroups start apart (W's pitch a multiple of 4 KB, and W larger than the caches)
+    changes no bit of the projection."""
+    from nanospec_amd import head
+
+    g = torch.Generator(device=DEV).manual_seed(7500 + n)
+    x = torch.randn((200, 2048), generator=g, device=DEV).bfloat16()
+    w = (0.05 * torch.randn((v, 2048), generator=g, device=DEV)).bfloat16()
+    assert torch.equal(head.lm_head_linear(x[:n], w), head.lm_head_linear(x, w)[:n])
