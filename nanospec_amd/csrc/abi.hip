@@ -422,8 +422,7 @@ int ns_lmhead_ce_kl_bwd(const void* hidden, int64_t ldh, const void* weight, int
   ns::SlotArgs a{labels, weights, nullptr, n, 1, c_ce, c_kl, inv_acc};
   const ns::TeacherSpec ts{teacher_args ? teacher_args->rows : nullptr, nt, teacher_args ? teacher_args->lse : nullptr};
   return hip_status(ns::lmhead_emit_dlogits(hidden, ldh, weight, ldw, markov, ldm, factors, teacher, t_dtype, ldt, d,
-                                            v, a, &ts, row_stats, dl, ldd, workspace, workspace_bytes,
-                                            reinterpret_cast<hipStream_t>(stream)),
+                                            v, a, &ts, row_stats, dl, ldd, workspace, reinterpret_cast<hipStream_t>(stream)),
                     "ns_lmhead_ce_kl_bwd");
 }
 

@@ -1,7 +1,7 @@
 // Fused LM head + draft objective on bf16 MFMA (gfx950, v_mfma_f32_32x32x16_bf16).
 //
 // Forward (nanospec/train.py:272-279 + objective.py:49-67), over windows of rows, so that at
-// most 2 GiB of logits are held at a time, whatever N is:
+// most 2 GiB of logits are held at a time, whatever N is (V up to 2^21):
 //   z^T tile = W_lm[v-tile] . hidden[t-tile]^T   (vocab on the MFMA M axis, tokens on N)
 //   pass 1 ("stats"): epilogue adds the Markov tile, reads the teacher tile and folds
 //     (max, sum-exp) of z and u plus A = sum exp(u - m_u)(u - z) into per-token running
@@ -1335,12 +1335,14 @@ HeadPlan head_plan(int64_t n, int64_t v) {
   return pl;
 }
 
-// The forward runs over windows of whole token tiles, so that the tile values pass 1 keeps for
-// pass 2 fit kZWindowBytes whatever N is (2,048 rows at V = 248,320): the
-// [N, V] logits beyond that never exist together.  Windows are of even size (all but the last the
-// same); pass 2 without kept values follows the same windows, so that both ways add every sum
-// in the same order.  At N = 4096 two windows cost pass 1 2% (31 vocab tiles a workgroup twice,
-// for 61 once).
+// Where pass 1's values are kept for pass 2 (keeps_tiles) the forward runs over windows of whole token
+// tiles, so that they fit kZWindowBytes whatever N is (2,048 rows at V = 248,320; a single token tile
+// past V = 2^21, where it alone is larger): the [N, V] logits beyond that never exist together.
+// Windows are of even size (all but the last the same); pass 2 without workspace for the values
+// follows the same windows, so that both ways add every sum in the same order.  At N = 4096 two
+// windows cost pass 1 2% (31 vocab tiles a workgroup twice, for 61 once).  Sizes whose values are
+// never kept, and pass 2 alone, take all rows at once (V = 248,320, d = 128, N = 16,384: the forward
+// 8.9 ms, in eight windows 9.4; pass 2 alone 4.7 and 5.0).
 constexpr int64_t kZWindowBytes = int64_t(2) << 30;
 
 int64_t window_rows(int64_t n, int64_t v) {
@@ -1739,7 +1741,7 @@ hipError_t lmhead_forward(const void* hidden, int64_t ldh, const void* weight, i
   // pass 2 reads pass 1's values when both run here and the workspace holds them
   const bool keep = drows || (parts == kHeadParts && keeps_tiles(a.n, v, d) &&
                               ws_bytes >= lmhead_workspace_bytes(a.n, v, d));
-  const int64_t rows = rows_per_window(a.n, v, ws_bytes);
+  const int64_t rows = drows || keeps_tiles(a.n, v, d) ? rows_per_window(a.n, v, ws_bytes) : a.n;
   for (int64_t r0 = 0; r0 < a.n; r0 += rows) {
     MarkovFactors f;
     const HeadArgs w = rows_of(x, &f, r0, a.n - r0 < rows ? a.n - r0 : rows);
@@ -1752,23 +1754,16 @@ hipError_t lmhead_forward(const void* hidden, int64_t ldh, const void* weight, i
 hipError_t lmhead_emit_dlogits(const void* hidden, int64_t ldh, const void* weight, int64_t ldw, const void* markov,
                                int64_t ldm, const MarkovFactors* factors, const void* teacher, int tdt, int64_t ldt,
                                int64_t d, int64_t v, const SlotArgs& a, const TeacherSpec* ts,
-                               const float* row_stats, void* dl, int64_t ldd, void* ws, size_t ws_bytes,
-                               hipStream_t st) {
+                               const float* row_stats, void* dl, int64_t ldd, void* ws, hipStream_t st) {
   if (a.n == 0) return hipSuccess;
   // pass 2 alone: the row log-normalisers come from the forward's row_stats, the accept
   // and KL partials it also forms go to the workspace and are not read
   const HeadArgs x = head_args(hidden, ldh, weight, ldw, markov, ldm, factors, teacher, tdt, ldt, d, v, a, ts, dl,
                                ldd, const_cast<float*>(row_stats));
-  const int64_t rows = rows_per_window(a.n, v, ws_bytes);
-  for (int64_t r0 = 0; r0 < a.n; r0 += rows) {
-    MarkovFactors f;
-    const HeadArgs xw = rows_of(x, &f, r0, a.n - r0 < rows ? a.n - r0 : rows);
-    const HeadPlan pl = head_plan(xw.a.n, v);
-    HeadWs w;
-    window_ws_layout(xw.a.n, pl.splits, ws, &w);
-    if (const hipError_t e = head_emit_window(head_params(xw, pl, w), pl, tdt, st); e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  const HeadPlan pl = head_plan(a.n, v);
+  HeadWs w;
+  window_ws_layout(a.n, pl.splits, ws, &w);
+  return head_emit_window(head_params(x, pl, w), pl, tdt, st);
 }
 
 size_t lmhead_bwd_workspace_bytes(int64_t n, int64_t v, int64_t d, int64_t r, bool norm) {

@@ -141,7 +141,7 @@ hipError_t lmhead_emit_dlogits(const void* hidden, int64_t ldh, const void* weig
                                const void* markov, int64_t ldm, const MarkovFactors* factors, const void* teacher,
                                int tdt, int64_t ldt, int64_t d, int64_t v, const SlotArgs& a,
                                const TeacherSpec* ts, const float* row_stats, void* dl, int64_t ldd, void* ws,
-                               size_t ws_bytes, hipStream_t st);
+                               hipStream_t st);
 // dh workspace; r > 0 adds the Markov column tiles' partials, norm the rms-norm
 // backward's column partials
 size_t lmhead_bwd_workspace_bytes(int64_t n, int64_t v, int64_t d, int64_t r = 0, bool norm = false);

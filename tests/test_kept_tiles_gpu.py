@@ -134,3 +134,22 @@ def test_few_rows_with_workgroups_started_apart(gpu_lib, n, v):
     x = torch.randn((200, 2048), generator=g, device=DEV).bfloat16()
     w = (0.05 * torch.randn((v, 2048), generator=g, device=DEV)).bfloat16()
     assert torch.equal(head.lm_head_linear(x[:n], w), head.lm_head_linear(x, w)[:n])
+
+
+def test_windows_only_where_values_are_kept(gpu_lib):
+    """Three windows of rows (V = 2^21) at a d whose values pass 2 reads; one launch of each pass where
+    they are not kept, and of pass 2 alone."""
+    from nanospec_amd import head
+    from nanospec_amd.config import Objective
+
+    n, v = 520, 1 << 21
+    for d, windows in ((320, 3), (64, 1)):
+        h, w, _, u, slots = synthetic.head_inputs(n, d, v, 7600 + d, DEV, ragged=True)
+        with _lib.KernelTimer() as t:
+            _, saved = head.lm_head_ce_kl_loss(h, w, u, slots, Objective(block_size=8), emit_dlogits=False)
+            torch.cuda.synchronize()
+        assert t.times["head_stats"][0] == windows and t.times["head_emit"][0] == windows
+        with _lib.KernelTimer() as t:
+            head._reemit_dlogits(saved, 1)
+            torch.cuda.synchronize()
+        assert t.times["head_emit"][0] == 1
