@@ -1338,9 +1338,11 @@ HeadPlan head_plan(int64_t n, int64_t v) {
 // Where pass 1's values are kept for pass 2 (keeps_tiles) the forward runs over windows of whole token
 // tiles, so that they fit kZWindowBytes whatever N is (2,048 rows at V = 248,320; a single token tile
 // past V = 2^21, where it alone is larger): the [N, V] logits beyond that never exist together.
-// Windows are of even size (all but the last the same); pass 2 without workspace for the values
-// follows the same windows, so that both ways add every sum in the same order.  At N = 4096 two
-// windows cost pass 1 2% (31 vocab tiles a workgroup twice, for 61 once).  Sizes whose values are
+// All but the last are the largest that fits, a multiple of four token tiles (whole XCD blocks, whole
+// rounds): windows of even size instead took six tiles twice at N = 3000 for eight and four, 8.53 ms
+// for 7.70 (d = 5120, V = 248,320), and 7.15 for 6.48 at N = 2560.  Pass 2 without workspace for the
+// values follows the same windows, so that both ways add every sum in the same order.  At N = 4096
+// two windows cost pass 1 2% (31 vocab tiles a workgroup twice, for 61 once).  Sizes whose values are
 // never kept, and pass 2 alone, take all rows at once (V = 248,320, d = 128, N = 16,384: the forward
 // 8.9 ms, in eight windows 9.4; pass 2 alone 4.7 and 5.0).
 constexpr int64_t kZWindowBytes = int64_t(2) << 30;
@@ -1351,8 +1353,7 @@ int64_t window_rows(int64_t n, int64_t v) {
   int64_t most = kZWindowBytes / (vt * kZTile * 4);   // token tiles
   if (most >= 4) most -= most % 4;                    // whole XCD blocks (4 x 8)
   if (most < 1) most = 1;
-  const int64_t windows = (tt + most - 1) / most;
-  return (tt + windows - 1) / windows * BN;
+  return (tt < most ? tt : most) * BN;
 }
 
 // Whether pass 2 reads pass 1's tile values (4 bytes written and 4 read per entry) rather than

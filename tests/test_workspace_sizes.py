@@ -37,3 +37,12 @@ def test_dh_splits_fill_the_xcds_evenly(lib, n, v, d):
     assert splits * tiles % 8 == 0 or splits < 8
     if v <= 4096:
         assert splits <= 24
+
+
+def test_windows_of_kept_values_are_the_largest_that_fit(lib):
+    """At V = 248,320 2 GiB hold eight token tiles' values: 3000 rows are windows of 2048 and 952 (whole
+    XCD blocks of four token tiles), not two of 1536."""
+    bytes_of = lambda n: lib.ns_workspace_bytes(_lib.NS_WS_LMHEAD, n, 248320, 5120)
+    values = 2048 * 248320 * 4
+    assert bytes_of(3000) >= values and bytes_of(2304) >= values
+    assert bytes_of(100000) < values + (1 << 28)
