@@ -20,6 +20,7 @@ HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))
 
 ABI_VERSION = 6
 NS_BF16, NS_F32 = 0, 1
+NS_ROW_NAN = -(1 << 63)
 NS_WS_LOGITS, NS_WS_LMHEAD, NS_WS_LMHEAD_BWD, NS_WS_FP8 = 0, 1, 2, 3
 NS_PART_STATS, NS_PART_EMIT = 1, 2
 NS_WS_RMS_NORM_BWD, NS_WS_LMHEAD_NORM_BWD, NS_WS_TEACHER_LOGITS, NS_WS_LMHEAD_MIN, NS_WS_LMHEAD_ROWS = 4, 5, 6, 7, 8

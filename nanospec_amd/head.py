@@ -205,11 +205,12 @@ def lm_head_ce_kl_loss(hidden, lm_head_weight, target_logits, prepared, objectiv
         raise ValueError("pass either markov_logits or markov factors, not both")
     wts, y, valid, k = _slot_inputs(prepared, n, device)
     if skip_masked_rows and markov is None and targs is None and emit_dlogits:
-        skipping = _forward_skipping_masked if _skips_on_values(n, vocab, d) else _forward_compact_rows
-        out = skipping(o, lm_head_weight, hidden.shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts, valid, k,
-                       accumulation_steps, device)
-        if out is not None:
-            return out
+        index, rows = _kept_rows(wts, valid, device)
+        if rows < n:   # else: the full pass
+            on_values = _skips_on_values(n, vocab, d) and _values_cost_less(n, rows, vocab, d)
+            skipping = _forward_skipping_masked if on_values else _forward_compact_rows
+            return skipping(o, lm_head_weight, hidden.shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts, valid, k,
+                            accumulation_steps, device, index, rows)
     metrics = torch.empty(6, dtype=torch.float32, device=device)
     row_stats = torch.empty((n, 8), dtype=torch.float32, device=device)
     dl = torch.empty((n, vocab), dtype=torch.bfloat16, device=device) if emit_dlogits else None
@@ -245,25 +246,42 @@ def _skips_on_values(n: int, vocab: int, d: int) -> bool:
     return d >= 896 or n * vocab <= 1 << 28
 
 
+def _values_cost_less(n: int, rows: int, vocab: int, d: int) -> bool:
+    """The same choice once it is known that ``rows`` of the rows are supervised: the values are
+    written for every row, the second GEMM (whole tiles of 256 rows) runs on those rows alone, after
+    the launches that gather them.  In microseconds, fitted to the times below (values / GEMM again,
+    V = 248,320 unless said): N = 4096, d = 896: 15% 3684 / 2991, 40% 3843 / 3768, 60% 3915 / 4383;
+    d = 2048: 15% 5224 / 4903, 25% 5282 / 5467; d = 5120: 2% 9305 / 9126, 7% 9593 / 9657; N = 2048, d =
+    1024: 25% 1906 / 1802, 40% 1965 / 2147; N = 1000, d = 1024: 2% 891 / 972; V = 128,000, N = 2000, d =
+    512: 25% 851 / 821, 40% 876 / 945."""
+    values = 1.1e-6 * n * vocab * (1 + 0.25 * rows / n)
+    again = 100 + 1e-6 * (-(-rows // 256) * 256) * vocab * (1.6 + 1.76e-3 * d)
+    return values <= again
+
+
+def _kept_rows(wts, valid, device):
+    """Each row's index among the supervised ones (-1: not one of them), and their count, read on the
+    host: it sizes dl."""
+    n = wts.shape[0]
+    index = torch.empty(n + 1, dtype=torch.int64, device=device)
+    status = _lib.load().ns_kept_rows(_lib.ptr(wts), _lib.ptr(valid), n, _lib.ptr(index), _lib.ptr(index[n:]),
+                                      _lib.stream(device))
+    _lib.check(status, "ns_kept_rows")
+    return index[:n], int(index[n])
+
+
 def _forward_skipping_masked(o, lm_head_weight, hidden_shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts, valid, k,
-                             accumulation_steps, device):
+                             accumulation_steps, device, index, rows):
     """lm_head_ce_kl_loss(skip_masked_rows=True): pass 1 on every row, dl formed from its values for
-    the supervised rows only, into a compact [rows, V] dl (ns_lmhead_ce_kl_fwd_rows) that is kept
+    the ``rows`` supervised rows only, into a compact [rows, V] dl (ns_lmhead_ce_kl_fwd_rows) that is kept
     with each row's index in it; the backward runs the dh GEMM on it and scatters dh among zero
     rows, and forms the [N, V] dl (zero rows between) only for a caller that asks for it
     (return_dlogits, final_norm).  An unsupervised row whose statistics are not finite has a NaN dl
-    and dh row: its index says so.  Returns None when every row is supervised."""
+    and dh row: its index says so."""
     lib = _lib.load()
     st = _lib.stream(device)
     n = h.shape[0]
     vocab, d = lm_head_weight.shape
-    index = torch.empty(n + 1, dtype=torch.int64, device=device)
-    _lib.check(lib.ns_kept_rows(_lib.ptr(wts), _lib.ptr(valid), n, _lib.ptr(index), _lib.ptr(index[n:]), st),
-               "ns_kept_rows")
-    rows = int(index[n])   # read on the host: it sizes dl
-    if rows == n:
-        return None
-    index = index[:n]
     metrics = torch.empty(6, dtype=torch.float32, device=device)
     row_stats = torch.empty((n, 8), dtype=torch.float32, device=device)
     dl = torch.empty((rows, vocab), dtype=torch.bfloat16, device=device)
@@ -282,11 +300,11 @@ def _forward_skipping_masked(o, lm_head_weight, hidden_shape, h, ldh, w, ldw, m,
 
 
 def _forward_compact_rows(o, lm_head_weight, hidden_shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts, valid, k,
-                          accumulation_steps, device):
+                          accumulation_steps, device, index, rows):
     """skip_masked_rows where a second GEMM over the kept rows costs less than pass 1's values
-    written and read (``_skips_on_values``): pass 1 on every row, then pass 2 on the rows whose dl
-    is not all zero (supervised, or with statistics that are not finite), their hidden and Markov
-    rows gathered into compact copies (ns_copy_rows), their teacher rows read in place."""
+    written and read (``_skips_on_values``, ``_values_cost_less``): pass 1 on every row, then pass 2 on the ``rows``
+    supervised ones, their hidden and Markov rows gathered into compact copies (ns_copy_rows),
+    their teacher rows read in place.  The outputs are ``_forward_skipping_masked``'s."""
     lib = _lib.load()
     st = _lib.stream(device)
     n = h.shape[0]
@@ -303,37 +321,33 @@ def _forward_compact_rows(o, lm_head_weight, hidden_shape, h, ldh, w, ldw, m, ld
 
     row_stats = torch.empty((n, 8), dtype=torch.float32, device=device)
     part(_lib.NS_PART_STATS, h, ldh, m, ldm, u, ldu, y, wts, n, None, row_stats)
-    # (the reference's dl of an unsupervised row is 0 * NaN there, its accept 0 * NaN)
-    need = (valid != 0) | (wts != 0) | ~torch.isfinite(row_stats[:, 0]) | ~torch.isfinite(row_stats[:, 1])
-    act = torch.nonzero(need).reshape(-1)   # reads the count on the host: it sizes the compacted pass
-    rows = act.numel()
-    dl = compact = None
-    if rows == n:
-        dl = torch.empty((n, vocab), dtype=torch.bfloat16, device=device)
-        part(_lib.NS_PART_EMIT, h, ldh, m, ldm, u, ldu, y, wts, n, dl, row_stats)
-    else:
-        hc = _lib.copy_rows(h, act, rows, torch.empty((rows, d), dtype=h.dtype, device=device))
-        mc = _lib.copy_rows(m, act, rows, torch.empty((rows, vocab), dtype=m.dtype, device=device)) \
-            if m is not None else None
-        # the teacher rows are read in place, gathered in the kernels' loads
-        targs = _lib.TeacherArgs(_lib.ptr(act), u.shape[0], None)
-        rs = row_stats.index_select(0, act)
-        dlc = torch.empty((rows, vocab), dtype=torch.bfloat16, device=device)
-        part(_lib.NS_PART_EMIT, hc, d, mc, vocab, u, ldu, y.index_select(0, act), wts.index_select(0, act), rows,
-             dlc, rs, targs)
-        del hc, mc
-        row_stats.index_copy_(0, act, rs)
-        row_stats[:, 4].masked_fill_(~need, 0.0)   # (accept_rate * valid) is 0 there either way
-        index = torch.full((n,), -1, dtype=torch.int64, device=device)
-        index.index_copy_(0, act, torch.arange(rows, dtype=torch.int64, device=device))
-        compact = _Compact(dlc, index)   # the [N, V] dl is formed only if a caller asks for it
+    act = torch.empty(rows + 1, dtype=torch.int64, device=device)   # the supervised rows, and one place more
+    act.scatter_(0, torch.where(index < 0, rows, index), torch.arange(n, dtype=torch.int64, device=device))
+    act = act[:rows]
+    hc = _lib.copy_rows(h, act, rows, torch.empty((rows, d), dtype=h.dtype, device=device))
+    mc = _lib.copy_rows(m, act, rows, torch.empty((rows, vocab), dtype=m.dtype, device=device)) \
+        if m is not None else None
+    # the teacher rows are read in place, gathered in the kernels' loads
+    targs = _lib.TeacherArgs(_lib.ptr(act), u.shape[0], None)
+    rs = row_stats.index_select(0, act)
+    dl = torch.empty((rows, vocab), dtype=torch.bfloat16, device=device)
+    part(_lib.NS_PART_EMIT, hc, d, mc, vocab, u, ldu, y.index_select(0, act), wts.index_select(0, act), rows, dl, rs,
+         targs)
+    del hc, mc
+    # an unsupervised row: accept 0, or NaN and a NaN dl row (the reference's 0 * NaN) where a
+    # log-normaliser is not finite
+    none = (index < 0) & torch.isfinite(row_stats[:, :2]).all(dim=1)
+    row_stats[:, 4] = torch.where(none, 0.0, float("nan"))
+    row_stats.index_copy_(0, act, rs)
+    index = torch.where((index < 0) & ~none, _lib.NS_ROW_NAN, index)
     metrics = torch.empty(6, dtype=torch.float32, device=device)
     status = lib.ns_objective_metrics(_lib.ptr(row_stats), _lib.ptr(wts), _lib.ptr(valid), n, k, float(o.ce),
                                       float(o.kl), _lib.ptr(metrics), st)
     _lib.check(status, "ns_objective_metrics")
     inputs = _HeadInputs(h, ldh, w, ldw, m, ldm, None, u, ldu, None, None, y, wts)
     shape = tuple(hidden_shape[:-1]) + (vocab,)
-    saved = HeadActivations(o, lm_head_weight, row_stats, dl, accumulation_steps, shape, None, inputs, compact)
+    saved = HeadActivations(o, lm_head_weight, row_stats, None, accumulation_steps, shape, None, inputs,
+                            _Compact(dl, index))
     return LossMetrics.from_buffer(metrics), saved
 
 

@@ -200,3 +200,24 @@ def test_both_ways_of_skipping_give_the_full_pass(gpu_lib, monkeypatch, on_value
     assert torch.isnan(dls[r]).all() and torch.isnan(dhs[r]).all()
     assert torch.equal(torch.isnan(dlf), torch.isnan(dls)) and torch.equal(torch.isnan(dhf), torch.isnan(dhs))
     assert torch.isnan(mf.accept_len_sum) and torch.isnan(ms.accept_len_sum)
+
+
+@pytest.mark.parametrize("on_values", [True, False])
+@pytest.mark.parametrize("supervised", [0, 1, 519, 520])
+def test_skipping_at_the_ends_of_the_supervised_count(gpu_lib, monkeypatch, on_values, supervised):
+    """No supervised row, one, all but one, all: both ways of skipping are the full pass."""
+    monkeypatch.setattr(head, "_skips_on_values", lambda n, v, d: on_values)
+    monkeypatch.setattr(head, "_values_cost_less", lambda n, rows, v, d: on_values)
+    n, d, v = 520, 320, 2184
+    hidden, weight, markov, teacher, slots = synthetic.head_inputs(n, d, v, 5711, DEV)
+    on = torch.zeros(n, dtype=torch.bool, device=DEV)
+    on[torch.randperm(n, generator=torch.Generator(device=DEV).manual_seed(supervised), device=DEV)[:supervised]] = True
+    slots.valid = on.view_as(slots.valid)
+    slots.weights = torch.where(slots.valid, slots.weights, torch.zeros_like(slots.weights))
+    full, skip = _both(hidden, weight, markov, teacher, slots, Objective(block_size=8))
+    if supervised:
+        _assert_same(full, skip, _masked(slots))
+    else:   # no row of dh to set a bar by: dl and dh are zero
+        assert torch.equal(full[1].row_stats[:, :4], skip[1].row_stats[:, :4])
+        for t in (full[2], skip[2], full[3], skip[3]):
+            assert torch.equal(t, torch.zeros_like(t))
