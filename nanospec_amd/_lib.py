@@ -202,10 +202,17 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
-def workspace(kind: int, n: int, v: int, d: int, device: torch.device) -> torch.Tensor:
+def workspace(kind: int, n: int, v: int, d: int, device: torch.device, least: int | None = None) -> torch.Tensor:
+    """A call's scratch.  ``least``: the kind of a smaller one that the call takes too, for a device
+    that has no room for the first."""
     nbytes = int(load().ns_workspace_bytes(kind, n, v, d))
     # torch's caching allocator returns 256-byte aligned blocks
-    return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
+    try:
+        return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        if least is None:
+            raise
+    return workspace(least, n, v, d, device)
 
 
 def rows_2d(t: torch.Tensor, cols: int) -> tuple[torch.Tensor, int]:

@@ -169,6 +169,9 @@ def lm_head_ce_kl_loss(hidden, lm_head_weight, target_logits, prepared, objectiv
     bit (accept rates may differ in their last bit where the kept rows go through a pass of their
     own).  Sizing dl reads the supervised rows' count on the host (one synchronisation), so this
     path cannot be captured into a graph; row statistics of the skipped rows carry accept_rate 0.
+
+    Memory: besides the outputs, up to 2 GiB of scratch for a window of pass 1's values, or a few MB
+    where the device has no room for it (pass 2 then runs the GEMM again, to the same bits).
     """
     o = objective
     if accumulation_steps < 1:
@@ -207,14 +210,17 @@ def lm_head_ce_kl_loss(hidden, lm_head_weight, target_logits, prepared, objectiv
     if skip_masked_rows and markov is None and targs is None and emit_dlogits:
         index, rows = _kept_rows(wts, valid, device)
         if rows < n:   # else: the full pass
-            on_values = _skips_on_values(n, vocab, d) and _values_cost_less(n, rows, vocab, d)
-            skipping = _forward_skipping_masked if on_values else _forward_compact_rows
-            return skipping(o, lm_head_weight, hidden.shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts, valid, k,
-                            accumulation_steps, device, index, rows)
+            args = (o, lm_head_weight, hidden.shape, h, ldh, w, ldw, m, ldm, u, ldu, y, wts, valid, k,
+                    accumulation_steps, device, index, rows)
+            out = None
+            if _skips_on_values(n, vocab, d) and _values_cost_less(n, rows, vocab, d):
+                out = _forward_skipping_masked(*args)
+            return out if out is not None else _forward_compact_rows(*args)
     metrics = torch.empty(6, dtype=torch.float32, device=device)
     row_stats = torch.empty((n, 8), dtype=torch.float32, device=device)
     dl = torch.empty((n, vocab), dtype=torch.bfloat16, device=device) if emit_dlogits else None
-    ws = _lib.workspace(_lib.NS_WS_LMHEAD, n, vocab, d, device)
+    # without room for a window's values pass 2 runs the GEMM again: the same bits
+    ws = _lib.workspace(_lib.NS_WS_LMHEAD, n, vocab, d, device, least=_lib.NS_WS_LMHEAD_MIN)
     tail = (_lib.ptr(u), _lib.dtype_code(u), ldu, ctypes.byref(targs) if targs is not None else None, _lib.ptr(y),
             _lib.ptr(wts), _lib.ptr(valid), n, d, vocab, k, float(o.ce), float(o.kl), 1.0 / accumulation_steps,
             _lib.ptr(dl), vocab, _lib.ptr(row_stats), _lib.ptr(metrics), _lib.ptr(ws), ws.numel(),
@@ -277,15 +283,18 @@ def _forward_skipping_masked(o, lm_head_weight, hidden_shape, h, ldh, w, ldw, m,
     with each row's index in it; the backward runs the dh GEMM on it and scatters dh among zero
     rows, and forms the [N, V] dl (zero rows between) only for a caller that asks for it
     (return_dlogits, final_norm).  An unsupervised row whose statistics are not finite has a NaN dl
-    and dh row: its index says so."""
+    and dh row: its index says so.  Returns None when the device has no room for the values."""
     lib = _lib.load()
     st = _lib.stream(device)
     n = h.shape[0]
     vocab, d = lm_head_weight.shape
+    try:
+        dl = torch.empty((rows, vocab), dtype=torch.bfloat16, device=device)
+        ws = _lib.workspace(_lib.NS_WS_LMHEAD_ROWS, n, vocab, d, device)
+    except torch.OutOfMemoryError:
+        return None
     metrics = torch.empty(6, dtype=torch.float32, device=device)
     row_stats = torch.empty((n, 8), dtype=torch.float32, device=device)
-    dl = torch.empty((rows, vocab), dtype=torch.bfloat16, device=device)
-    ws = _lib.workspace(_lib.NS_WS_LMHEAD_ROWS, n, vocab, d, device)
     status = lib.ns_lmhead_ce_kl_fwd_rows(
         _lib.ptr(h), ldh, _lib.ptr(w), ldw, _lib.ptr(m), ldm, _lib.ptr(u), _lib.dtype_code(u), ldu, None, _lib.ptr(y),
         _lib.ptr(wts), _lib.ptr(valid), n, d, vocab, k, float(o.ce), float(o.kl), 1.0 / accumulation_steps,
