@@ -107,8 +107,12 @@ int ns_abi_version(void);
 /* Thread-local text of the last non-zero status. */
 const char* ns_last_error(void);
 
-/* Scratch bytes an entry point of `kind` needs (NS_WS_*); d is ignored by
- * NS_WS_LOGITS and NS_WS_TEACHER_LOGITS, v by NS_WS_RMS_NORM_BWD. */
+/* Scratch bytes for an entry point of `kind` (NS_WS_*); d is ignored by
+ * NS_WS_LOGITS and NS_WS_TEACHER_LOGITS, v by NS_WS_RMS_NORM_BWD.  NS_WS_LOGITS and
+ * NS_WS_RMS_NORM_BWD never shrink as n grows, so a workspace for a caller's largest n takes every
+ * smaller one; the others depend on n's split into tiles and are asked for each n.  The dh GEMM's
+ * kinds hold the K splits that are fastest: its entry points also take less, down to
+ * min(16, four rounds of workgroups) splits' partials, with as many splits as fit. */
 size_t ns_workspace_bytes(int kind, int64_t n, int64_t v, int64_t d);
 
 /* Forward objective over given logits (objective.py:49-67) plus, when dl is not

@@ -469,11 +469,11 @@ int ns_lmhead_bwd(const void* dl, int64_t ldd, const void* weight, int64_t ldw, 
   if ((rc = check_matrix(dh, n, d, lddh, "dh"))) return rc;
   if (!aligned(dl) || !aligned(weight) || !aligned(dh) || ldd % 8 || ldw % 8 || lddh % 4)
     return fail(NS_EALIGN, "dh GEMM needs 16-byte aligned base pointers and rows");
-  const size_t need = ns::lmhead_bwd_workspace_bytes(n, v, d);
+  const size_t need = ns::lmhead_bwd_required_bytes(n, v, d);
   if (n > 0 && (!workspace || workspace_bytes < need))
     return fail(NS_EWORKSPACE, "workspace of %zu bytes required (got %zu)", need, workspace_bytes);
   if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return fail(NS_EALIGN, "workspace must be 256-byte aligned");
-  return hip_status(ns::lmhead_backward(dl, ldd, weight, ldw, dh, lddh, n, v, d, workspace,
+  return hip_status(ns::lmhead_backward(dl, ldd, weight, ldw, dh, lddh, n, v, d, workspace, workspace_bytes,
                                         reinterpret_cast<hipStream_t>(stream)),
                     "ns_lmhead_bwd");
 }
@@ -508,7 +508,7 @@ int ns_lmhead_markov_bwd(const void* dl, int64_t ldd, const void* weight, int64_
       !aligned(w2_grad) || ldd % 8 || ldw % 8 || ldw1 % 8 || ldw2 % 8 || lddh % (norm ? 8 : 4) || ldg1 % 8 ||
       ldg2 % 8)
     return fail(NS_EALIGN, "Markov backward needs 16-byte aligned base pointers and rows");
-  const size_t need = ns::markov_bwd_workspace_bytes(n, v, d, r);
+  const size_t need = ns::markov_bwd_required_bytes(n, v, d, r);
   if (n > 0 && (!workspace || workspace_bytes < need))
     return fail(NS_EWORKSPACE, "workspace of %zu bytes required (got %zu)", need, workspace_bytes);
   if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return fail(NS_EALIGN, "workspace must be 256-byte aligned");
@@ -570,12 +570,12 @@ int ns_lmhead_norm_bwd(const void* dl, int64_t ldd, const void* weight, int64_t 
   if (dh && (rc = check_matrix(dh, n, d, lddh, "dh"))) return rc;
   if (!aligned(dl) || !aligned(weight) || !aligned(dh) || ldd % 8 || ldw % 8 || (dh && lddh % 8))
     return fail(NS_EALIGN, "dh GEMM needs 16-byte aligned base pointers and rows");
-  const size_t need = ns::lmhead_bwd_workspace_bytes(n, v, d, 0, true);
+  const size_t need = ns::lmhead_bwd_required_bytes(n, v, d, 0, true);
   if (n > 0 && (!workspace || workspace_bytes < need))
     return fail(NS_EWORKSPACE, "workspace of %zu bytes required (got %zu)", need, workspace_bytes);
   if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return fail(NS_EALIGN, "workspace must be 256-byte aligned");
   return hip_status(ns::lmhead_backward_ext(dl, ldd, weight, ldw, nullptr, 0, 0, dh, lddh, nullptr, &nb, n, v, d,
-                                            workspace, reinterpret_cast<hipStream_t>(stream)),
+                                            workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream)),
                     "ns_lmhead_norm_bwd");
 }
 

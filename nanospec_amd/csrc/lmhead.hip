@@ -24,6 +24,7 @@
 // stage buffers, persistent workgroups that walk a contiguous vocab range with per-token
 // running statistics, and a workgroup -> tile map that puts the workgroups sharing a W
 // stream on the same XCD (shared L2).
+#include <climits>
 #include <type_traits>
 
 #include "ns_gemm.h"
@@ -1465,7 +1466,17 @@ int bwd_splits(int64_t n, int64_t v, int64_t d, int tiles, int kt_total, int cus
   return ks;
 }
 
-BwdPlan bwd_plan(int64_t n, int64_t v, int64_t d, int64_t r = 0) {
+// K splits of the Markov column tiles, which run after the dh tiles as one extra round: enough to give
+// every CU one (each then covers a fraction of V), at least the dh count.
+int markov_splits(int tiles2, int ks, int kt_total, int cus) {
+  int ks2 = tiles2 > 0 ? (cus + tiles2 - 1) / tiles2 : 1;
+  if (ks2 < ks) ks2 = ks;
+  if (ks2 > 64) ks2 = 64;
+  return ks2 > kt_total ? kt_total : ks2;
+}
+
+// most_splits: of dh, where the workspace holds no more
+BwdPlan bwd_plan(int64_t n, int64_t v, int64_t d, int64_t r = 0, int most_splits = INT_MAX) {
   BwdPlan pl;
   pl.mt = (int)((n + BM - 1) / BM);
   pl.ct = (int)((d + BN - 1) / BN);
@@ -1473,21 +1484,19 @@ BwdPlan bwd_plan(int64_t n, int64_t v, int64_t d, int64_t r = 0) {
   pl.kt_total = (int)((v + BK - 1) / BK);
   const int tiles = pl.mt * pl.ct;
   const int cus = device_cus();
-  const int ks = tiles > 0 ? bwd_splits(n, v, d, tiles, pl.kt_total, cus) : 1;   // no tiles: nothing launches
+  int ks = tiles > 0 ? bwd_splits(n, v, d, tiles, pl.kt_total, cus) : 1;   // no tiles: nothing launches
+  if (ks > most_splits) {
+    ks = most_splits;
+    while (ks > kNumXcd && (int64_t)tiles * ks % kNumXcd) --ks;
+  }
   pl.ksplit = ks;
   pl.grid_main = tiles * ks;
-  // Markov tiles run after the dh tiles as one extra round: enough K splits to give
-  // every CU one (each then covers a fraction of V), at least the dh count
   pl.ksplit2 = 0;
   pl.grid = pl.grid_main;
   if (pl.ct2 > 0) {
     const int tiles2 = pl.mt * pl.ct2;
-    int ks2 = tiles2 > 0 ? (cus + tiles2 - 1) / tiles2 : 1;
-    if (ks2 < ks) ks2 = ks;
-    if (ks2 > 64) ks2 = 64;
-    if (ks2 > pl.kt_total) ks2 = pl.kt_total;
-    pl.ksplit2 = ks2;
-    pl.grid += tiles2 * ks2;
+    pl.ksplit2 = markov_splits(tiles2, ks, pl.kt_total, cus);
+    pl.grid += tiles2 * pl.ksplit2;
   }
   // XCD block (dh_kernel's tile order): xa * xb = CUs per XCD, xa | mt, xb | ct, whole
   // rounds on every XCD; the smallest xa + xb.  Failing whole rounds, the grid of blocks is
@@ -1767,22 +1776,51 @@ hipError_t lmhead_emit_dlogits(const void* hidden, int64_t ldh, const void* weig
   return head_emit_window(head_params(x, pl, w), pl, tdt, st);
 }
 
+namespace {
+
+size_t bwd_partial_bytes(int64_t n, int64_t d, int64_t r, int ks, int ks2) {
+  return align_up((size_t)ks * n * d * sizeof(float), 256) + align_up((size_t)ks2 * n * r * sizeof(float), 256);
+}
+
+// The partials of a plan with at most `most` splits of dh.
+size_t bwd_bytes(const BwdPlan& pl, int64_t n, int64_t d, int64_t r, int most) {
+  const int ks = pl.ksplit < most ? pl.ksplit : most;
+  return bwd_partial_bytes(n, d, r, ks, r > 0 ? markov_splits(pl.mt * pl.ct2, ks, pl.kt_total, device_cus()) : 0);
+}
+
+// The splits every workspace must hold: four rounds of workgroups, at most 16.
+int bwd_least_splits(const BwdPlan& pl) {
+  const int tiles = pl.mt * pl.ct, rounds = 4 * device_cus();
+  const int ks = tiles > 0 ? (rounds + tiles - 1) / tiles : 1;
+  return ks > 16 ? 16 : ks;
+}
+
+}  // namespace
+
 size_t lmhead_bwd_workspace_bytes(int64_t n, int64_t v, int64_t d, int64_t r, bool norm) {
+  return bwd_bytes(bwd_plan(n, v, d, r), n, d, r, INT_MAX) + (norm ? norm_bwd_workspace_bytes(n, d) : 0);
+}
+
+size_t lmhead_bwd_required_bytes(int64_t n, int64_t v, int64_t d, int64_t r, bool norm) {
   const BwdPlan pl = bwd_plan(n, v, d, r);
-  return align_up((size_t)pl.ksplit * n * d * sizeof(float), 256) +
-         align_up((size_t)pl.ksplit2 * n * r * sizeof(float), 256) + (norm ? norm_bwd_workspace_bytes(n, d) : 0);
+  return bwd_bytes(pl, n, d, r, bwd_least_splits(pl)) + (norm ? norm_bwd_workspace_bytes(n, d) : 0);
 }
 
 hipError_t lmhead_backward(const void* dl, int64_t ldd, const void* weight, int64_t ldw, void* dh, int64_t lddh,
-                           int64_t n, int64_t v, int64_t d, void* ws, hipStream_t st) {
-  return lmhead_backward_ext(dl, ldd, weight, ldw, nullptr, 0, 0, dh, lddh, nullptr, nullptr, n, v, d, ws, st);
+                           int64_t n, int64_t v, int64_t d, void* ws, size_t ws_bytes, hipStream_t st) {
+  return lmhead_backward_ext(dl, ldd, weight, ldw, nullptr, 0, 0, dh, lddh, nullptr, nullptr, n, v, d, ws, ws_bytes,
+                             st);
 }
 
 hipError_t lmhead_backward_ext(const void* dl, int64_t ldd, const void* weight, int64_t ldw, const void* w2,
                                int64_t ldw2, int64_t r, void* dh, int64_t lddh, float* dprev, const NormBwd* norm,
-                               int64_t n, int64_t v, int64_t d, void* ws, hipStream_t st) {
+                               int64_t n, int64_t v, int64_t d, void* ws, size_t ws_bytes, hipStream_t st) {
   if (n == 0 || d == 0) return hipSuccess;
-  const BwdPlan pl = bwd_plan(n, v, d, r);
+  BwdPlan pl = bwd_plan(n, v, d, r);
+  const size_t b_norm = norm ? norm_bwd_workspace_bytes(n, d) : 0;
+  int most = pl.ksplit;
+  while (most > 1 && bwd_bytes(pl, n, d, r, most) + b_norm > ws_bytes) --most;
+  if (most < pl.ksplit) pl = bwd_plan(n, v, d, r, most);
   BwdParams p = {};
   p.dl = static_cast<const uint16_t*>(dl);
   p.weight = static_cast<const uint16_t*>(weight);

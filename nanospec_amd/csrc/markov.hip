@@ -363,8 +363,8 @@ struct MarkovWs {
   float* piece;                // [n, r] run-piece sums
 };
 
-size_t markov_ws_layout(int64_t n, int64_t v, int64_t d, int64_t r, void* base, MarkovWs* w) {
-  const size_t b_dh = align_up(lmhead_bwd_workspace_bytes(n, v, d, r, true), 256);
+// Everything but the dh GEMM's partials (b_dh bytes, at the workspace's start).
+size_t markov_ws_layout(int64_t n, int64_t r, size_t b_dh, void* base, MarkovWs* w) {
   const size_t b_dp = align_up((size_t)n * r * sizeof(float), 256);
   const size_t b_e = align_up((size_t)n * r * 2, 256);
   const size_t b_k = align_up((size_t)sort_padded(n) * sizeof(uint64_t), 256);
@@ -377,13 +377,17 @@ size_t markov_ws_layout(int64_t n, int64_t v, int64_t d, int64_t r, void* base, 
     w->keys_b = reinterpret_cast<uint64_t*>(p); p += b_k;
     w->piece = reinterpret_cast<float*>(p);
   }
-  return b_dh + b_dp + b_e + 2 * b_k + b_dp;
+  return b_dp + b_e + 2 * b_k + b_dp;
 }
 
 }  // namespace
 
 size_t markov_bwd_workspace_bytes(int64_t n, int64_t v, int64_t d, int64_t r) {
-  return markov_ws_layout(n, v, d, r, nullptr, nullptr);
+  return align_up(lmhead_bwd_workspace_bytes(n, v, d, r, true), 256) + markov_ws_layout(n, r, 0, nullptr, nullptr);
+}
+
+size_t markov_bwd_required_bytes(int64_t n, int64_t v, int64_t d, int64_t r) {
+  return align_up(lmhead_bwd_required_bytes(n, v, d, r, true), 256) + markov_ws_layout(n, r, 0, nullptr, nullptr);
 }
 
 hipError_t markov_backward(const void* dl, int64_t ldd, const void* weight, int64_t ldw, const MarkovFactors& f,
@@ -391,11 +395,14 @@ hipError_t markov_backward(const void* dl, int64_t ldd, const void* weight, int6
                            int64_t ldg2, int64_t n, int64_t v, int64_t d, void* ws, size_t ws_bytes, hipStream_t st) {
   const int64_t r = f.r;
   MarkovWs w;
-  markov_ws_layout(n, v, d, r, ws, &w);
+  const size_t full = align_up(lmhead_bwd_workspace_bytes(n, v, d, r, true), 256);
+  size_t b_dh = (ws_bytes - markov_ws_layout(n, r, 0, nullptr, nullptr)) & ~size_t(255);
+  if (b_dh > full) b_dh = full;
+  markov_ws_layout(n, r, b_dh, ws, &w);
   hipError_t e;
   // dh (or the rms-norm backward) and d(previous) in one GEMM
   if ((e = lmhead_backward_ext(dl, ldd, weight, ldw, f.w2, f.ldw2, r, dh, lddh, w.dprev, norm, n, v, d, w.dh_ws,
-                               st)) != hipSuccess)
+                               b_dh, st)) != hipSuccess)
     return e;
   if (n == 0) return hipSuccess;
   {
@@ -439,7 +446,6 @@ hipError_t markov_backward(const void* dl, int64_t ldd, const void* weight, int6
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL(markov_runs_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, w.keys_a, n, v, r, w.piece,
                      static_cast<uint16_t*>(w1_grad), ldg1);
-  (void)ws_bytes;
   return hipGetLastError();
 }
 

@@ -203,8 +203,17 @@ int norm_rows_per_block(int64_t n) {
 }
 
 size_t norm_bwd_workspace_bytes(int64_t n, int64_t d) {
+  // the column partials of any number of rows up to n (n's own are fewer where it takes more rows a
+  // workgroup)
   const int rows = norm_rows_per_block(n);
-  return align_up((size_t)((n + rows - 1) / rows) * d * sizeof(float), 256);
+  int64_t blocks = (n + rows - 1) / rows;
+  for (const int64_t below : {1023, 2047, 8191})
+    if (n > below) {
+      const int r = norm_rows_per_block(below);
+      const int64_t b = (below + r - 1) / r;
+      blocks = blocks > b ? blocks : b;
+    }
+  return align_up((size_t)blocks * d * sizeof(float), 256);
 }
 
 hipError_t rms_norm_forward(const void* x, int64_t ldx, const void* weight, int64_t n, int64_t d, float eps,

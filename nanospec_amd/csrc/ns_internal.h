@@ -145,18 +145,22 @@ hipError_t lmhead_emit_dlogits(const void* hidden, int64_t ldh, const void* weig
 // dh workspace; r > 0 adds the Markov column tiles' partials, norm the rms-norm
 // backward's column partials
 size_t lmhead_bwd_workspace_bytes(int64_t n, int64_t v, int64_t d, int64_t r = 0, bool norm = false);
+// what a call needs at least: with less than the above it takes as many K splits as fit
+size_t lmhead_bwd_required_bytes(int64_t n, int64_t v, int64_t d, int64_t r = 0, bool norm = false);
 hipError_t lmhead_backward(const void* dl, int64_t ldd, const void* weight, int64_t ldw, void* dh,
-                           int64_t lddh, int64_t n, int64_t v, int64_t d, void* ws, hipStream_t st);
+                           int64_t lddh, int64_t n, int64_t v, int64_t d, void* ws, size_t ws_bytes,
+                           hipStream_t st);
 // dh = dl . weight and, when r > 0, dprev = dl . w2 (fp32 [N, r], row stride r) in the same
 // GEMM.  With norm, the split-K reduction is the rms-norm backward: dx and the norm weight's
 // gradient are written, and dh only if dh is not NULL.
 hipError_t lmhead_backward_ext(const void* dl, int64_t ldd, const void* weight, int64_t ldw, const void* w2,
                                int64_t ldw2, int64_t r, void* dh, int64_t lddh, float* dprev, const NormBwd* norm,
-                               int64_t n, int64_t v, int64_t d, void* ws, hipStream_t st);
+                               int64_t n, int64_t v, int64_t d, void* ws, size_t ws_bytes, hipStream_t st);
 // Markov-head backward (markov.hip): dh (or, with norm, dx and the norm weight's gradient),
 // w2_grad = dl^T . w1[prev] (overwritten) and w1_grad.index_add_(prev, dl . w2)
 // (accumulated, deterministic order)
 size_t markov_bwd_workspace_bytes(int64_t n, int64_t v, int64_t d, int64_t r);
+size_t markov_bwd_required_bytes(int64_t n, int64_t v, int64_t d, int64_t r);
 hipError_t markov_backward(const void* dl, int64_t ldd, const void* weight, int64_t ldw, const MarkovFactors& f,
                            void* dh, int64_t lddh, const NormBwd* norm, void* w1_grad, int64_t ldg1, void* w2_grad,
                            int64_t ldg2, int64_t n, int64_t v, int64_t d, void* ws, size_t ws_bytes, hipStream_t st);

@@ -74,9 +74,17 @@ struct StreamWs {
   float* zy;
 };
 
+// Partials of pass 1 that a workspace holds: at least n * stream_splits(n, v), and never fewer for more
+// rows (n * ceil(kStatsGroups / n) rises and falls with n), so that a workspace sized for a caller's
+// largest n takes every smaller one.
+static int64_t stats_parts(int64_t n, int64_t v) {
+  const int64_t least = n * splits_for(v, kStatsElems, kStatsMaxSplits);
+  const int64_t most = n * splits_for(v, kStatsMinElems, kStatsMaxSplits), few = kStatsGroups + 2 * n;
+  return least > few ? least : most < few ? most : few;
+}
+
 static size_t stream_ws_layout(int64_t n, int64_t v, void* base, StreamWs* out) {
-  const int S = stream_splits(n, v);
-  const size_t b1 = align_up((size_t)n * S * sizeof(RowPart), 256);
+  const size_t b1 = align_up((size_t)stats_parts(n, v) * sizeof(RowPart), 256);
   const size_t b2 = align_up((size_t)n * emit_splits(v) * sizeof(float), 256);
   const size_t b3 = align_up((size_t)n * sizeof(float), 256);
   if (out) {

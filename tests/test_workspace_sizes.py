@@ -46,3 +46,12 @@ def test_windows_of_kept_values_are_the_largest_that_fit(lib):
     values = 2048 * 248320 * 4
     assert bytes_of(3000) >= values and bytes_of(2304) >= values
     assert bytes_of(100000) < values + (1 << 28)
+
+
+@pytest.mark.parametrize("kind,v,d", [
+    (_lib.NS_WS_LOGITS, 248320, 0), (_lib.NS_WS_LOGITS, 50001, 0), (_lib.NS_WS_LOGITS, 8192, 0),
+    (_lib.NS_WS_LOGITS, 1, 0), (_lib.NS_WS_RMS_NORM_BWD, 0, 5120), (_lib.NS_WS_RMS_NORM_BWD, 0, 8),
+])
+def test_a_workspace_for_the_largest_n_takes_every_smaller_one(lib, kind, v, d):
+    sizes = [lib.ns_workspace_bytes(kind, n, v, d) for n in [*range(2300), 4096, 8191, 8192, 8193, 20000]]
+    assert all(a <= b for a, b in zip(sizes, sizes[1:]))
