@@ -8,7 +8,8 @@ input that is already resident in HBM.
 
     python bench.py [--steps K] [--warmup W] [--config c1|c2|c2x|c3|c4]
 
-Prints ONE JSON line.  By default the headline is C2 (the configuration the metric is
+Prints ONE JSON line of a few KB on stdout, and the same with every kernel's figures on stderr before
+it.  By default the headline is C2 (the configuration the metric is
 quoted on) and C1, C3, C4 and C2X follow in the same process under "secondary".  One GPU only: ``--gpus N`` with N > 1 exits with a
 message (the path is data-parallel over slots; the library has no collectives).
 """
@@ -1002,6 +1003,39 @@ def measure(wl, args, config_name):
     return out
 
 
+def _short(x):
+    """Floats to six significant digits, through lists and dicts."""
+    if isinstance(x, float):
+        return float(f"{x:.6g}")
+    if isinstance(x, dict):
+        return {k: _short(v) for k, v in x.items()}
+    if isinstance(x, (list, tuple)):
+        return [_short(v) for v in x]
+    return x
+
+
+def _workload_summary(r):
+    """A workload's kernels as milliseconds a step, and its rooflines as their fractions."""
+    out = {"kernels_ms": {k: i["step_ms"] for k, i in r["kernels"].items()},
+           "roofline_fracs": {k: i["frac"] for k, i in r["rooflines"].items()}}
+    return {k: v for k, v in out.items() if v}
+
+
+def summary(line):
+    """The printed line: what a reader of the metric needs, in a few KB (a reader that keeps only the
+    end of the output still has all of it).  The whole measurement goes to stderr."""
+    detail = ("rooflines", "kernels", "inputs_sha256", "library_ceilings", "secondary")
+    out = {k: v for k, v in line.items() if k not in detail}
+    out.update(_workload_summary(line))
+    if line["secondary"]:
+        out["secondary"] = {name: {"value": r["value"], "ms_per_step": r["ms_per_step"], "steps": r["steps"],
+                                   "N": r["config"]["N"], "dtype": r["dtype"], "step_roofline": r["step_roofline"],
+                                   "roofline": {k: r["roofline"][k] for k in ("kernel", "bound", "achieved", "unit",
+                                                                             "frac")}}
+                            for name, r in line["secondary"].items()}
+    return _short(out)
+
+
 def main():
     args = parse()
     if args.traffic_from:
@@ -1097,7 +1131,8 @@ def main():
         "host": {"cpu_model": cpu_model(), "cpu_count": os.cpu_count()},
         "device": torch.cuda.get_device_name(device),
     }
-    print(json.dumps(line), flush=True)
+    print(json.dumps(line), file=sys.stderr, flush=True)
+    print(json.dumps(summary(line)), flush=True)
 
 
 if __name__ == "__main__":

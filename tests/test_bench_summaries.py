@@ -134,3 +134,41 @@ def test_stats_summary_launch_column(tmp_path):
         w.writerow([DH, 2, 20_000_000, 10_000_000, 50.0])
     text = bench.stats_summary(str(d), "c2", "cmd")
     assert "| dh_gemm | 2 | 20.000 | 10.0000 | 50.0 |" in text
+
+
+def _measured(config, kernels):
+    roof = {"bound": "mfma", "achieved": 1234.5678901234567, "peak": 2500.0, "unit": "TFLOP/s",
+            "frac": 0.49382715604938266, "dtype": "bf16", "kernel": "head_stats", "kernel_mean_ms": 4.1234567890123,
+            "traffic": 4101323885, "traffic_source": "profiles/lmhead_c2_traffic.md",
+            "traffic_GBs": 2444.1320616019693, "traffic_frac_hbm": 0.3055165077002462, "clock_GHz": 1.689,
+            "mfma_busy": 0.6513, "mfma_per_clock": 0.6513, "mfma_source": "profiles/lmhead_c2_mfma.md"}
+    return {"value": 225731.12345678912, "unit": "slots/s", "steps": 20, "warmup": 3, "warmup_steps_run": 14,
+            "ms_per_step": 18.146234567891234, "dtype": "bf16", "roofline": dict(roof), "wall_s": 0.3629246913578247,
+            "config": {"workload": config + " LM-head GEMM + Markov addend + CE+KL+accept fwd, dl + dhidden bwd",
+                       "N": 4096, "d": 5120, "V": 248320, "K": 8, "gamma": 4.0, "global_batch": 4096, "seq_len": None,
+                       "parallelism": "single GPU"},
+            "step_roofline": {"algorithmic_TFLOPs": 1147.9123456789123, "mfma_frac": 0.45916493827156492},
+            "kernels": {f"kernel_name_{i}": {"launches": 40, "mean_ms": 1.2345678901234567, "step_ms": 2.469135780246913,
+                                             "window": "5 steps after", "algorithmic_GBs": 5755.79184913229}
+                        for i in range(kernels)},
+            "rooflines": {f"kernel_name_{i}": dict(roof) for i in range(4)}}
+
+
+def test_printed_line_keeps_the_headline_within_a_few_kilobytes():
+    import json
+
+    res = _measured("C2", 16)
+    line = {"metric": bench.METRIC, "n_gpus": 1, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
+            "data": "synthetic", **res, "cpu_baseline": {"value": 21.123456789, "sample": "1536 rows " * 20},
+            "library_ceilings": {"gemm": {"TFLOPs": 1234.5678}}, "inputs_sha256": {f"t{i}": "0" * 64 for i in range(9)},
+            "secondary": {f"c{i}": _measured(f"C{i}", 20) for i in range(5)},
+            "host": {"cpu_model": "x" * 60, "cpu_count": 128}, "device": "AMD Instinct MI355X"}
+    assert len(json.dumps(line)) > 8192
+    out = bench.summary(line)
+    assert len(json.dumps(out)) < 5000
+    for k in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+              "vs_baseline", "dtype", "data", "config", "roofline"):
+        assert k in out
+    assert out["value"] == 225731.0 and out["ms_per_step"] == 18.1462 and out["config"] == line["config"]
+    assert set(out["secondary"]) == set(line["secondary"])
+    assert out["roofline"]["frac"] == 0.493827 and out["kernels_ms"]["kernel_name_3"] == 2.46914
