@@ -997,7 +997,7 @@ def measure(wl, args, config_name):
     out = {"value": value, "unit": "slots/s", "steps": args.steps, "warmup": args.warmup, "warmup_steps_run": warm,
            "ms_per_step": ms_per_step, "dtype": wl["dtype"], "config": wl["config"], "roofline": roof,
            "step_roofline": step_roof, "kernels": kernels, "wall_s": wall}
-    # every kernel the north star sets a target for: the HBM stream kernels and the GEMMs
+    # every kernel with a target: the HBM stream kernels and the GEMMs
     out["rooflines"] = {k: roofline(k) for k in kernels
                         if k in wl["kernel_flops"] or k in fp8_flops or k in wl.get("stream_kernels", ())}
     return out
@@ -1117,7 +1117,7 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": res["dtype"],
-        "data": "synthetic (seeded; distributions of BASELINE.json configs)",
+        "data": "synthetic (seeded inputs of the benchmark's shapes, random-init weights)",
         "config": res["config"],
         "roofline": res["roofline"],
         "step_roofline": res["step_roofline"],

@@ -1,4 +1,4 @@
-"""The north star's dhidden bar, applied per row (shared by the GPU tests).
+"""The dhidden bar, applied per row (shared by the GPU tests).
 
 On every row: max |dh - dh_ref| <= 2e-2 of that row's largest |dh_ref| and cosine >= 0.9999;
 a row whose reference is exactly zero (a masked slot) is exactly zero.  This is the

@@ -11,7 +11,7 @@ oracle (objective.py:49-80 with ops.py:183-200 for C4's teacher and train.py:302
   Accept rates are then 0.5-0.9, and KL = A/s_u - lse_u + lse_z cancels terms of 12-17 down
   to about 0.1.  The same 1e-4 bar applies.
 
-dhidden bar (north star): on every row, max |dh - dh_ref| <= 2e-2 max |dh_ref| and cosine
+dhidden bar: on every row, max |dh - dh_ref| <= 2e-2 max |dh_ref| and cosine
 >= 0.9999.  dl bar: one bf16 ulp plus the fp32 evaluation error where (c_ce + c_kl) p and
 c_kl t cancel.
 """

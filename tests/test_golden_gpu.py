@@ -1,5 +1,5 @@
 """The HIP library against the torch-made golden fixtures of the head region
-(tests/golden/head_small.npz, norm_small.npz), at the north-star tolerances: metrics within
+(tests/golden/head_small.npz, norm_small.npz), at the path's stated tolerances: metrics within
 1e-4 relative, dl within one bf16 ulp plus fp32 evaluation error, dh cosine >= 0.9999 and
 max error <= 2e-2 of max |dh|, Markov gradients within bf16 output rounding, rms_norm within
 one bf16 ulp (forward) and its propagation (backward)."""

@@ -1,7 +1,7 @@
 """GPU parity of the fused LM-head path (ns_lmhead_ce_kl_fwd, ns_lmhead_bwd,
 ns_lmhead_linear) against the CPU oracle.
 
-Tolerances (north star): loss, ce, kl, accept_len within 1e-4 relative of the
+Tolerances: loss, ce, kl, accept_len within 1e-4 relative of the
 fp32 objective; the label pick exact in index; dhidden per row max error <= 2e-2
 of the row's max|dh| and cosine >= 0.9999; dl within one bf16 ulp plus fp32
 evaluation error.  The benchmark sizes are in test_fullsize_gpu.py.

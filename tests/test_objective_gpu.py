@@ -1,7 +1,7 @@
 """GPU parity of the logits-level objective (ns_ce_kl_logits_fwd / _bwd) against
 the CPU oracle and the library-made golden vectors.
 
-Tolerances (north star): loss, ce, kl, accept_len within 1e-4 relative of the
+Tolerances: loss, ce, kl, accept_len within 1e-4 relative of the
 fp32 objective; token-index work (label pick) exact; dl within one bf16 ulp of
 the exact value (bf16 logits) or 1e-4 relative (fp32 logits).
 """
