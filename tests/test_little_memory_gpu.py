@@ -48,10 +48,13 @@ def test_no_room_for_the_kept_values(gpu_lib, room, monkeypatch, form):
                                       for t in (h, w, markov, u, want, factors)]
     kinds, workspace = [], _lib.workspace
     monkeypatch.setattr(_lib, "workspace", lambda kind, *a, **kw: kinds.append(kind) or workspace(kind, *a, **kw))
-    # room for dl of all rows and the compact one, not for the values beside a dl
+    # room for dl of all rows and the compact one, dh's partials and 40 MB of small blocks (the segments
+    # of 20 MB that they come in): with the compact dl alone allocated 216 MB are left, not the
+    # 268 MB of the values
     assert gpu_lib.ns_workspace_bytes(_lib.NS_WS_LMHEAD, n, v, d) > 4 * n * v
-    dl = 2 * n * v
-    room((dl + dl * 5 // 8 if form == "skip" else dl) + (40 << 20))
+    dl, partials = 2 * n * v, gpu_lib.ns_workspace_bytes(_lib.NS_WS_LMHEAD_BWD, n, v, d)
+    assert dl + partials + (40 << 20) < 4 * n * v
+    room((dl + dl * 5 // 8 if form == "skip" else dl) + partials + (40 << 20))
     got = _step((h, w, markov, u, slots, head.MarkovFactors(*factors)), form)
     assert _lib.NS_WS_LMHEAD_MIN in kinds
     for a, b in zip(want, got):
