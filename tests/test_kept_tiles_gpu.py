@@ -96,6 +96,42 @@ def test_several_windows_of_rows(gpu_lib):
         assert float(stats[r, 4]) == pytest.approx(float(torch.minimum(p, t).sum()), rel=1e-4)
 
 
+@pytest.mark.parametrize("kind", [_lib.NS_WS_LMHEAD, _lib.NS_WS_LMHEAD_MIN])
+@pytest.mark.parametrize("form", ["dense", "gathered", "lse", "fp32", "fp32_lse", "factored", "no_dl"])
+def test_each_window_is_a_call_of_its_rows(gpu_lib, form, kind):
+    """Every operand moves on with the window: three windows of 256, 256 and 8 rows (V = 2^21) give the
+    row statistics and dl of three calls on those rows, bit for bit."""
+    n, d, v, step = 520, 320, 1 << 21, 256
+    h, w, markov, u, slots = synthetic.head_inputs(n, d, v, 7350, DEV, ragged=True)
+    slots.target_ids[40, 3] = -100
+    rows = lse = factors = None
+    if form != "dense":
+        markov = None
+    if form.startswith("fp32"):
+        u = u.float()
+    if form.endswith("lse"):
+        lse = torch.stack([torch.logsumexp(x.double(), -1) for x in u]).float()
+    if form == "gathered":
+        rows = torch.randint(0, n, (n,), device=DEV)
+        rows[300] = n            # outside: that row's teacher is NaN
+        rows[515] = -1
+    if form == "factored":
+        factors = synthetic.markov_factors(n, v, 64, 7351, DEV)
+        factors[0][400] = v      # outside: that row's logits are NaN
+    _, stats, dl = _forward(gpu_lib, kind, h, w, u, slots, markov=markov, factors=factors, rows=rows, lse=lse,
+                            want_dl=form != "no_dl")
+    for r0 in range(0, n, step):
+        r = slice(r0, min(r0 + step, n))
+        b = slice(r0 // 8, r.stop // 8)
+        part = synthetic.Slots(slots.weights[b], slots.target_ids[b], slots.valid[b])
+        _, s, x = _forward(gpu_lib, kind, h[r], w, u if rows is not None else u[r], part,
+                           markov=None if markov is None else markov[r],
+                           factors=None if factors is None else (factors[0][r], *factors[1:]),
+                           rows=None if rows is None else rows[r], lse=None if lse is None else lse[r],
+                           want_dl=form != "no_dl")
+        _assert_same([stats[r], None if dl is None else dl[r]], [s, x])
+
+
 @pytest.mark.parametrize("n", [1, 7, 32, 33, 64, 65, 100, 128])
 @pytest.mark.parametrize("v,d", [(8, 64), (8456, 320), (131336, 128)])
 def test_few_rows_projection(gpu_lib, n, v, d):

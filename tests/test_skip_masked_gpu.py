@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from nanospec_amd import head, synthetic
+from nanospec_amd import _lib, head, synthetic
 from nanospec_amd.config import Objective
 
 from dh_bar import assert_dh_rows
@@ -221,3 +221,39 @@ def test_skipping_at_the_ends_of_the_supervised_count(gpu_lib, monkeypatch, on_v
         assert torch.equal(full[1].row_stats[:, :4], skip[1].row_stats[:, :4])
         for t in (full[2], skip[2], full[3], skip[3]):
             assert torch.equal(t, torch.zeros_like(t))
+
+
+@pytest.mark.parametrize("form", ["plain", "dense", "fp32"])
+def test_skipping_over_several_windows(gpu_lib, monkeypatch, form):
+    """V = 2^21: windows of 256, 256 and 8 rows.  dl's rows are numbered over all of them, and an
+    unsupervised row with a NaN in the second and in the third is marked there: the full pass."""
+    monkeypatch.setattr(head, "_skips_on_values", lambda n, v, d: True)
+    monkeypatch.setattr(head, "_values_cost_less", lambda n, rows, v, d: True)
+    n, d, v = 520, 320, 1 << 21
+    hidden, weight, mk, teacher, slots = synthetic.head_inputs(n, d, v, 5721, DEV, ragged=True)
+    slots.valid[[40, 64], 5:] = False   # rows 325 and 517 are not supervised
+    slots.weights[[40, 64], 5:] = 0.0
+    if form == "fp32":
+        teacher = teacher.float()
+    mk = mk if form == "dense" else None
+    with _lib.KernelTimer() as t:
+        full, skip = _both(hidden, weight, mk, teacher, slots, Objective(block_size=8))
+    assert t.times["head_emit"][0] == 6   # three windows of each pass
+    masked = _masked(slots)
+    _assert_same(full, skip, masked)
+    del full, skip
+    hidden = hidden.clone()
+    bad = [325, 517]
+    assert bool(masked[bad].all())
+    hidden[bad, 9] = float("nan")
+    (_, sf, dhf, dlf), (_, ss, dhs, dls) = _both(hidden, weight, mk, teacher, slots, Objective(block_size=8))
+    ok = torch.ones(n, dtype=torch.bool, device=DEV)
+    ok[bad] = False
+    for a, b in ((dlf, dls), (sf.row_stats[:, :4], ss.row_stats[:, :4])):
+        a, b = a.reshape(n, -1), b.reshape(n, -1)
+        assert torch.equal(a[ok], b[ok])
+        assert torch.equal(torch.isnan(a[bad]), torch.isnan(b[bad]))
+    assert torch.isnan(dls.reshape(n, -1)[bad]).all() and torch.isnan(dhs.reshape(n, -1)[bad]).all()
+    assert_dh_rows(dhs.reshape(n, -1)[ok].float().cpu().numpy(), dhf.reshape(n, -1)[ok].float().cpu().numpy())
+    keep = ok & masked.to(DEV)
+    assert not dhs.reshape(n, -1)[keep].any()
