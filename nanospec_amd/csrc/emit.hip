@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256) void emit_rows_kernel(const float* __restrict_
                                                         int64_t rows, int vt, int splits, int64_t n,
                                                         float* __restrict__ row_stats, int64_t* __restrict__ drows,
                                                         int64_t ndl) {
-  extern __shared__ float sh[];   // [LSE ? 2 : 1][splits][16]
+  extern __shared__ float sh[];   // [LSE ? 2 : 1][splits][kSumRows]
   const int rl = threadIdx.x % kSumRows, l = threadIdx.x / kSumRows;
   const int64_t r = (int64_t)blockIdx.x * kSumRows + rl;
   const int64_t rc = r < n ? r : n - 1;

@@ -11,9 +11,10 @@
 //   pass 2 ("emit"): p = exp(z - LSE_z), t = exp(u - LSE_u), accumulates sum min(p, t) and
 //     writes dl = (w/acc)[(c_ce + c_kl) p - c_kl t - c_ce e_y] as bf16.  With workspace for
 //     one window's values pass 1 keeps its fp32 tiles there (kKeepZ: 4 bytes per entry written
-//     beside the epilogue, 3% of pass 1) and pass 2 streams over them (emit.hip); without, it
-//     runs the GEMM again (head_kernel<EMIT>).  At N = 4096, d = 5120, V = 248,320: both passes
-//     16.5 ms with the GEMM twice, 10.4 ms with the values kept (two windows).
+//     beside the epilogue) and pass 2 streams over them (emit.hip); without, it runs the GEMM
+//     again (head_kernel<EMIT>).  At N = 4096, d = 5120, V = 248,320: both passes 16.5 ms with the
+//     GEMM twice, 10.4 ms with the values kept, though pass 1 takes 8.95 ms for 8.17 (2% of it two
+//     windows for one).
 // Backward (train.py:302): dh = dl . W_lm as a long-K (K = V) split-K MFMA GEMM with a
 // fixed-order fp32 reduction of the split partials.
 //
@@ -1357,12 +1358,6 @@ int64_t window_rows(int64_t n, int64_t v) {
   return (tt < most ? tt : most) * BN;
 }
 
-// Whether pass 2 reads pass 1's tile values (4 bytes written and 4 read per entry) rather than
-// running the GEMM again (2 d operations per entry).  Both passes in microseconds, kept against
-// GEMM again, V = 248,320 unless said: N = 3500: d = 128 2557 / 2219, 256 2761 / 2663, 384
-// 2972 / 3030, 512 3296 / 3452; N = 448: 128 360 / 359, 256 382 / 417; N = 2048, V = 32,000:
-// 128 198 / 183, 256 210 / 211; N = 56: 128 147 / 200; N = 64, V = 8192, d = 64: 40 / 55.  The
-// fewer the values, the more of them the Infinity Cache (256 MB) still holds for pass 2.
 // Whether few rows' pass 1 and projection take thin.hip's kernel.  Projections here / with 256-token
 // tiles in microseconds, V = 248,320 unless said: d = 5120: n = 8 430 / 638, 64 470 / 635, 128
 // 527 / 649; d = 512: n = 8 45 / 86, 128 79 / 97; V = 8192, d = 5120: n = 8 49 / 92, 64 73 / 92;
@@ -1371,6 +1366,12 @@ int64_t window_rows(int64_t n, int64_t v) {
 // 118 / 92.
 bool thin_rows(int64_t n, int64_t v) { return n <= 64 || (n <= kThinRows && (v + BM - 1) / BM > kThinWide); }
 
+// Whether pass 2 reads pass 1's tile values (4 bytes written and 4 read per entry) rather than
+// running the GEMM again (2 d operations per entry).  Both passes in microseconds, kept against
+// GEMM again, V = 248,320 unless said: N = 3500: d = 128 2557 / 2219, 256 2761 / 2663, 384
+// 2972 / 3030, 512 3296 / 3452; N = 448: 128 360 / 359, 256 382 / 417; N = 2048, V = 32,000:
+// 128 198 / 183, 256 210 / 211; N = 56: 128 147 / 200; N = 64, V = 8192, d = 64: 40 / 55.  The
+// fewer the values, the more of them the Infinity Cache (256 MB) still holds for pass 2.
 bool keeps_tiles(int64_t n, int64_t v, int64_t d) {
   const int64_t entries = n * v;
   return d >= (entries <= (int64_t(1) << 25) ? 64 : entries <= (int64_t(1) << 27) ? 192 : 320);
