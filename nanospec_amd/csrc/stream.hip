@@ -52,13 +52,14 @@ static int splits_for(int64_t v, int64_t elems, int max_splits) {
 }
 
 // Pass 1's ranges: kStatsElems entries, shorter (down to kStatsMinElems) where the rows alone
-// leave CUs without workgroups: N = 224, V = 50,001 (fp32) ran 448 workgroups, 42 us with element loads, now
-// 2912 with vectors 20 us.
+// leave CUs without workgroups, as many as bring them to kStatsGroups: N = 224, V = 50,001 (fp32) ran
+// 448 workgroups, 42 us with element loads, now 2240 with vectors 20 us.  Exactly as many: lengths cut down
+// to a whole number of entries gave nearly every row one range more, and rows that already fill the chip
+// another part of a round (N = 324, V = 200,001, bf16: 8 ranges 141.9 us, the 7 of more rows 133.4).
 int stream_splits(int64_t n, int64_t v) {
+  const int least = splits_for(v, kStatsElems, kStatsMaxSplits), most = splits_for(v, kStatsMinElems, kStatsMaxSplits);
   const int64_t want = n > 0 ? (kStatsGroups + n - 1) / n : 1;
-  int64_t elems = want > 0 ? v / want : v;
-  elems = elems < kStatsMinElems ? kStatsMinElems : elems > kStatsElems ? kStatsElems : elems;
-  return splits_for(v, elems, kStatsMaxSplits);
+  return want < least ? least : want > most ? most : (int)want;
 }
 
 static int emit_splits(int64_t v) { return splits_for(v, kEmitElems, kEmitMaxSplits); }
@@ -79,7 +80,7 @@ struct StreamWs {
 // largest n takes every smaller one.
 static int64_t stats_parts(int64_t n, int64_t v) {
   const int64_t least = n * splits_for(v, kStatsElems, kStatsMaxSplits);
-  const int64_t most = n * splits_for(v, kStatsMinElems, kStatsMaxSplits), few = kStatsGroups + 2 * n;
+  const int64_t most = n * splits_for(v, kStatsMinElems, kStatsMaxSplits), few = kStatsGroups + n;
   return least > few ? least : most < few ? most : few;
 }
 

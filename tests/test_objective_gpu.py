@@ -304,3 +304,17 @@ def test_power_of_two_steps_rescale_the_emitted_dl(gpu_lib, dtype):
     _, s3 = nobj.ce_kl_loss(z, u, slots, o, accumulation_steps=3)
     torch.cuda.synchronize()
     assert torch.equal(dl3, nobj.ce_kl_backward(s3, 3))
+
+
+@pytest.mark.parametrize("v", [200001, 142689])
+def test_split_ranges_of_rows_that_fill_the_chip(gpu_lib, v):
+    """Pass 1 cuts rows that fill the chip by themselves into no more ranges than those of a larger batch
+    (324 rows x 7 ranges are 2268 workgroups): their statistics are the same bits in both."""
+    n, rows = 1000, 2048 // (-(-v // 32768)) // 4 * 4 + 32
+    assert rows < n
+    z, u, slots = synthetic.logits_inputs(n, v, 1900, DEV, k=4)
+    few = synthetic.Slots(slots.weights[: rows // 4], slots.target_ids[: rows // 4], slots.valid[: rows // 4])
+    o = Objective(block_size=4)
+    _, whole = nobj.ce_kl_loss(z, u, slots, o)
+    _, part = nobj.ce_kl_loss(z[:rows], u[:rows], few, o)
+    assert torch.equal(part.row_stats[:, :4], whole.row_stats[:rows, :4])
