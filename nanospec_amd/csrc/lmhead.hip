@@ -1430,17 +1430,20 @@ struct BwdPlan {
 // 1, 2, .. kMaxRounds whole ones, and the largest the sum takes in four groups (kFourGroups), the one of
 // least cost in units of a K entry of one 256 x 256 tile (24 ns: 0.77 us a 32-K stage): rounds x (a
 // workgroup's share of K + kTileCost for its first fills and its partial tile's store, about 15 us)
-// + the partials' write and sum (8 bytes per entry and split at 5.6 TB/s) + kSplitCost a split (0.1 us,
-// the sum's chain) + kGroupsCost (2.4 us) past four groups, where a norm that follows needs a launch more.
+// + the partials' write and sum (8 bytes per entry and split at 4.8 TB/s) + kSplitCost a split (7 ns)
+// + kGroupsCost per entry (7 ps) past four groups, whose sum reads shorter pieces of the partials.
 // Counts whose workgroups are not a multiple of the XCDs are rounded down to one: such a grid is not
 // laid out by XCD (N = 700, d = 1024, V = 32,000: 12 tiles x 20 splits 59 us, x 21 84 us).
 //
 // Against at most 16 splits for four rounds (dh in us): V = 248,320, d = 5120: N = 224 12 splits 596
 // for 764, N = 700 4 splits 1496 for 1649; V = 32,000, d = 1024: N = 8 24 for 41; V = 8192, d = 2048: N
 // = 1000 49 for 72.  Against whole rounds only (V = 4096): d = 256, N = 224 64 splits 23.3, 24 splits
-// 20.1; d = 1024, N = 64 64 splits 22.3, 24 splits 18.7.
+// 20.1.  Few rows take most of a round, as their partials are small: d = 256, N = 1 V = 65,536 128 splits
+// 19.5, 256 16.4; V = 4096 24 splits 12.8, 64 11.4.  Over 876 sizes (N 1 to 3000, d 256 to 5120, V 4096 to
+// 248,320, with and without a norm) the count taken is 2.1% faster in the mean than the better of those two
+// rules' and more than 5% slower at 9 sizes (at most 9%).
 constexpr int kMaxRounds = 6, kFourGroups = 24;
-constexpr double kTileCost = 640, kPartialCost = 6e-5, kSplitCost = 4, kGroupsCost = 100;
+constexpr double kTileCost = 640, kPartialCost = 7e-5, kSplitCost = 0.3, kGroupsCost = 3e-4;
 
 int bwd_splits(int64_t n, int64_t v, int64_t d, int tiles, int kt_total, int cus) {
   int step = 1;   // splits whose workgroups are a multiple of the XCDs
@@ -1454,7 +1457,7 @@ int bwd_splits(int64_t n, int64_t v, int64_t d, int tiles, int kt_total, int cus
     if (c == last) return;
     last = c;
     const double cost = (double)(((int64_t)tiles * c + cus - 1) / cus) * ((double)v / c + kTileCost) + c * per_split +
-                        (c > kFourGroups ? kGroupsCost : 0);
+                        (c > kFourGroups ? (double)n * d * kGroupsCost : 0);
     if (ks == 0 || cost < best || (cost == best && c < ks)) {
       best = cost;
       ks = c;

@@ -30,13 +30,22 @@ def test_few_rows_have_at_most_256_vocab_splits(lib, v):
 def test_dh_splits_fill_the_xcds_evenly(lib, n, v, d):
     """dh's grid is laid out by XCD only when its workgroups are a multiple of the 8 XCDs: no plan
     leaves it short of that (the workspace is its splits' fp32 partials), and no small vocabulary is cut
-    into shares that cost more to sum than they save."""
+    into shares that cost more to sum than they save (few rows' sum costs next to nothing)."""
     tiles = -(-n // 256) * -(-d // 256)
     splits = lib.ns_workspace_bytes(_lib.NS_WS_LMHEAD_BWD, n, v, d) // (4 * n * d)
     assert 1 <= splits <= -(-v // 64)
     assert splits * tiles % 8 == 0 or splits < 8
-    if v <= 4096:
+    if v <= 4096 and n >= 224:
         assert splits <= 24
+
+
+@pytest.mark.parametrize("v", [4096, 16384, 65536])
+@pytest.mark.parametrize("n", [1, 4, 8])
+def test_dh_of_few_rows_takes_most_of_a_round(lib, n, v):
+    """Few rows' partials are small, so that more workgroups pay: one for each K stage (64 entries), or
+    for more than half of the CUs."""
+    splits = lib.ns_workspace_bytes(_lib.NS_WS_LMHEAD_BWD, n, v, 256) // (4 * n * 256)
+    assert splits == v // 64 or splits > 128
 
 
 def test_windows_of_kept_values_are_the_largest_that_fit(lib):
